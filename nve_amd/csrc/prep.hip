@@ -104,11 +104,9 @@ __device__ __forceinline__ float load_w(const void* w, size_t i) {
   return load_act<WDT>(w, i);
 }
 
-// Q4 modes: plain (from_f32 / from_compact), AWQ (from_compact_awq: column j scaled by
-// awq[j] before the plain block quantizer, src/quantize.rs:271-306) and AWQ k-quant
-// (from_compact_awq_kquant, 308-346: the block scale is the candidate amax_c / 7 over
-// the 8 largest |v| that minimises sum_j awq[j]^2 (v_j - deq_j)^2, 741-793).
-enum { Q4_PLAIN = 0, Q4_AWQ = 1, Q4_AWQ_KQUANT = 2 };
+// Q4 modes: plain (from_f32 / from_compact) and AWQ (from_compact_awq: column j scaled by
+// awq[j] before the plain block quantizer, src/quantize.rs:271-306).
+enum { Q4_PLAIN = 0, Q4_AWQ = 1 };
 
 template <int WDT, int MODE>
 __global__ __launch_bounds__(256) void q4_quantize_kernel(const void* __restrict__ w, uint8_t* __restrict__ nib,
@@ -121,7 +119,6 @@ __global__ __launch_bounds__(256) void q4_quantize_kernel(const void* __restrict
 #pragma unroll
   for (int i = 0; i < 32; ++i) v[i] = load_w<WDT>(w, blk * 32 + i);
   const int col0 = MODE == Q4_PLAIN ? 0 : (int)(blk % (size_t)bpr) * 32;
-  float scale;
   if constexpr (MODE != Q4_PLAIN) {
 #pragma unroll
     for (int t = 0; t < 8; ++t) {
@@ -139,57 +136,10 @@ __global__ __launch_bounds__(256) void q4_quantize_kernel(const void* __restrict
         awq_inv[col0 + i] = fabsf(sc) > 1e-10f ? 1.0f / sc : 0.0f;
       }
   }
-  if constexpr (MODE == Q4_AWQ_KQUANT) {
-    // Candidate c is the c-th largest |v| (descending sort, src/quantize.rs:746-751):
-    // the element whose rank -- the count of larger values plus equal values at lower
-    // indices -- is c.  Equal values are interchangeable, so any sort order gives the
-    // same candidates (finite inputs).
-    float a[32];
+  float amax = 0.0f;
 #pragma unroll
-    for (int i = 0; i < 32; ++i) a[i] = fabsf(v[i]);
-    float cand[8];
-#pragma unroll
-    for (int c = 0; c < 8; ++c) cand[c] = 0.0f;
-#pragma unroll
-    for (int i = 0; i < 32; ++i) {
-      int r = 0;
-#pragma unroll
-      for (int j = 0; j < 32; ++j) r += (a[j] > a[i]) | (j < i && a[j] == a[i]);
-#pragma unroll
-      for (int c = 0; c < 8; ++c) cand[c] = r == c ? a[i] : cand[c];
-    }
-    float best_scale = 0.0f, best_err = 3.40282347e38f;  // f32::MAX
-    bool live = true;
-#pragma unroll
-    for (int c = 0; c < 8; ++c) {
-      live = live && !(cand[c] < 1e-10f);  // the reference breaks at the first tiny candidate
-      if (live) {
-        const float cs = cand[c] / 7.0f;
-        const float ci = 1.0f / cs;
-        float err = 0.0f;
-#pragma unroll
-        for (int j = 0; j < 32; ++j) {
-          int q = rust_as_i8(roundf(v[j] * ci));
-          q = q < -8 ? -8 : (q > 7 ? 7 : q);
-          const float aj = awq[col0 + j];
-          // (imp * d) * d + err, each product and the sum rounded on its own (Rust
-          // does not contract to FMA)
-          const float d = __fsub_rn(v[j], __fmul_rn((float)q, cs));
-          err = __fadd_rn(err, __fmul_rn(__fmul_rn(__fmul_rn(aj, aj), d), d));
-        }
-        if (err < best_err) {
-          best_err = err;
-          best_scale = cs;
-        }
-      }
-    }
-    scale = best_scale;
-  } else {
-    float amax = 0.0f;
-#pragma unroll
-    for (int i = 0; i < 32; ++i) amax = fmaxf(amax, fabsf(v[i]));
-    scale = amax > 0.0f ? amax / 7.0f : 0.0f;
-  }
+  for (int i = 0; i < 32; ++i) amax = fmaxf(amax, fabsf(v[i]));
+  const float scale = amax > 0.0f ? amax / 7.0f : 0.0f;
   const float inv = scale > 0.0f ? 1.0f / scale : 0.0f;
   int q[32];
 #pragma unroll
@@ -211,6 +161,142 @@ __global__ __launch_bounds__(256) void q4_quantize_kernel(const void* __restrict
   }
   ((uint4*)nib)[blk] = make_uint4(d[0], d[1], d[2], d[3]);
   scales[blk] = scale;
+}
+
+// AWQ k-quant (from_compact_awq_kquant, src/quantize.rs:308-346): the block scale is the
+// candidate amax_c / 7 over the 8 largest |v| that minimises sum_j awq[j]^2 (v_j - deq_j)^2
+// (first minimum, 741-793).
+//
+// VALU-bound: each block tries 8 scales on 32 values.  A lane owns one block, and the 64
+// lanes of a wave take 64 rows of one block column, so the column's 32 factors are
+// wave-uniform (scalar loads); the four waves take adjacent columns and the results leave
+// through LDS as whole 64-byte pieces of a row.  The candidates come from sorting networks
+// (four sorted octets merged to the top 8, about 250 min / max; counting every value's rank
+// took 3,000 operations), and a trial is seven operations on |v|: the error of -v against -q
+// is that of v against q, so the sign only sets the clamp.  3B gate (8192 x 3072 bf16):
+// 60 us, 124 us with one thread per block, rank counting and signed integer codes.
+constexpr float kHalfDown = 0x1.fffffep-2f;  // the float below 1/2: floor(y + it) == round(y) for 0 <= y < 4096
+// (checked over every float of the range), and above that the clamp decides
+
+__device__ __forceinline__ void ce_desc(float& a, float& b) {
+  const float hi = fmaxf(a, b);
+  b = fminf(a, b);
+  a = hi;
+}
+// sort descending: 8 values (Batcher's odd-even merge, 19 exchanges)
+__device__ __forceinline__ void sort8_desc(float (&c)[8]) {
+  constexpr int n[19][2] = {{0, 1}, {2, 3}, {4, 5}, {6, 7}, {0, 2}, {1, 3}, {4, 6}, {5, 7}, {1, 2}, {5, 6},
+                            {0, 4}, {1, 5}, {2, 6}, {3, 7}, {2, 4}, {3, 5}, {1, 2}, {3, 4}, {5, 6}};
+#pragma unroll
+  for (int i = 0; i < 19; ++i) ce_desc(c[n[i][0]], c[n[i][1]]);
+}
+// a <- the 8 largest of a and b (both descending), descending
+__device__ __forceinline__ void top8_desc(float (&a)[8], const float (&b)[8]) {
+#pragma unroll
+  for (int i = 0; i < 8; ++i) a[i] = fmaxf(a[i], b[7 - i]);  // bitonic
+#pragma unroll
+  for (int h = 4; h >= 1; h >>= 1)
+#pragma unroll
+    for (int i = 0; i < 8; ++i)
+      if (!(i & h)) ce_desc(a[i], a[i + h]);
+}
+
+template <int WDT>
+__global__ __launch_bounds__(256) void q4_kquant_kernel(const void* __restrict__ w, uint8_t* __restrict__ nib,
+                                                        float* __restrict__ scales, int N,
+                                                        const float* __restrict__ awq, float* __restrict__ awq_inv,
+                                                        int bpr, int col_groups) {
+#pragma clang fp contract(off)  // fused only where written: |v| / scale is rounded before the half is added
+  __shared__ uint4 s_nib[64][5];
+  __shared__ float s_sc[64][5];
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int cg = blockIdx.x % col_groups;
+  const int row0 = (int)(blockIdx.x / col_groups) * 64;
+  const int col = 4 * cg + wave;
+  if (col < bpr) {  // wave-uniform
+    const int row = min(row0 + lane, N - 1);
+    const size_t e0 = ((size_t)row * bpr + col) * 32;
+    const float* __restrict__ aw = awq + 32 * col;
+    float v[32];
+#pragma unroll
+    for (int i = 0; i < 32; ++i) v[i] = load_w<WDT>(w, e0 + i) * aw[i];
+    // the workgroups of row 0 also write the inverse scales (|s| > 1e-10 ? 1/s : 0)
+    if (awq_inv && row0 == 0 && lane < 32) {
+      const float sc = aw[lane];
+      awq_inv[32 * col + lane] = fabsf(sc) > 1e-10f ? 1.0f / sc : 0.0f;
+    }
+    // Candidate c is the c-th largest |v| (descending sort, src/quantize.rs:746-751); equal
+    // values are interchangeable.  A block with a NaN or an infinity has no finite error for
+    // any candidate: scale 0.
+    float cand[8], other[8];
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+#pragma unroll
+      for (int i = 0; i < 8; ++i) other[i] = fabsf(v[8 * t + i]);
+      sort8_desc(other);
+      if (t == 0) {
+#pragma unroll
+        for (int i = 0; i < 8; ++i) cand[i] = other[i];
+      } else {
+        top8_desc(cand, other);
+      }
+    }
+    float cs[8], ci[8], err[8];
+#pragma unroll
+    for (int c = 0; c < 8; ++c) {
+      cs[c] = cand[c] / 7.0f;
+      ci[c] = 1.0f / cs[c];
+      err[c] = 0.0f;
+    }
+#pragma unroll
+    for (int j = 0; j < 32; ++j) {
+      const float a = fabsf(v[j]), lim = v[j] < 0.0f ? 8.0f : 7.0f;
+      const float imp = aw[j] * aw[j];
+#pragma unroll
+      for (int c = 0; c < 8; ++c) {
+        // |q| = min(round(|v| / scale), 8 or 7); the difference and the sum are one rounding
+        // each
+        const float q = fminf(floorf(a * ci[c] + kHalfDown), lim);
+        const float d = fmaf(-q, cs[c], a);
+        err[c] = fmaf(imp * d, d, err[c]);
+      }
+    }
+    float scale = 0.0f, best_err = 3.40282347e38f;  // f32::MAX
+#pragma unroll
+    for (int c = 0; c < 8; ++c) {
+      // the reference stops at the first candidate below 1e-10 (they descend)
+      const bool take = !(cand[c] < 1e-10f) && err[c] < best_err;
+      best_err = take ? err[c] : best_err;
+      scale = take ? cs[c] : scale;
+    }
+    const float inv = scale > 0.0f ? 1.0f / scale : 0.0f;
+    float q[32];
+#pragma unroll
+    for (int i = 0; i < 32; ++i) {
+      const float y = fabsf(v[i]) * inv;
+      float r = fminf(floorf(y + kHalfDown), v[i] < 0.0f ? 8.0f : 7.0f);
+      r = y == y ? r : 0.0f;  // `as i8` of a NaN
+      q[i] = 8.0f + copysignf(r, v[i]);
+    }
+    uint32_t d[4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      d[k] = 0;
+#pragma unroll
+      for (int t = 0; t < 4; ++t)  // GPU byte j = element j | element j+16 << 4
+        d[k] |= (uint32_t)(q[4 * k + t] + 16.0f * q[4 * k + t + 16]) << (8 * t);
+    }
+    s_nib[lane][wave] = make_uint4(d[0], d[1], d[2], d[3]);
+    s_sc[lane][wave] = scale;
+  }
+  __syncthreads();
+  const int r = threadIdx.x >> 2, c = threadIdx.x & 3;
+  if (row0 + r < N && 4 * cg + c < bpr) {
+    const size_t blk = (size_t)(row0 + r) * bpr + 4 * cg + c;
+    ((uint4*)nib)[blk] = s_nib[r][c];
+    scales[blk] = s_sc[r][c];
+  }
 }
 
 // ---- reference CPU Q4_0 bytes -> GPU layout (extract_for_gpu on the device) -------
@@ -385,25 +471,31 @@ hipError_t launch_q8_rows(const void* x, int xdt, int M, int K, int8_t* xq, uint
   return hipGetLastError();
 }
 
+template <int DT>
+static void launch_q4_dt(const void* w, size_t nblocks, int bpr, const float* awq, int kquant, uint8_t* nib,
+                         float* scales, float* awq_inv, hipStream_t stream) {
+  const unsigned grid = (unsigned)((nblocks + 255) / 256);
+  if (!awq) {
+    hipLaunchKernelGGL((nve::q4_quantize_kernel<DT, nve::Q4_PLAIN>), dim3(grid), dim3(256), 0, stream, w, nib, scales,
+                       nblocks, awq, awq_inv, bpr);
+  } else if (kquant) {
+    const int N = (int)(nblocks / bpr), cg = (bpr + 3) / 4;
+    hipLaunchKernelGGL(nve::q4_kquant_kernel<DT>, dim3((unsigned)((N + 63) / 64) * cg), dim3(256), 0, stream, w, nib,
+                       scales, N, awq, awq_inv, bpr, cg);
+  } else {
+    hipLaunchKernelGGL((nve::q4_quantize_kernel<DT, nve::Q4_AWQ>), dim3(grid), dim3(256), 0, stream, w, nib, scales,
+                       nblocks, awq, awq_inv, bpr);
+  }
+}
+
 hipError_t launch_q4_quantize_awq(const void* w, int wdt, size_t nblocks, int bpr, const float* awq, int kquant,
                                   uint8_t* nib, float* scales, float* awq_inv, hipStream_t stream) {
-  const unsigned grid = (unsigned)((nblocks + 255) / 256);
-#define NVE_Q4Q(DT, MODE)                                                                                      \
-  hipLaunchKernelGGL((nve::q4_quantize_kernel<DT, MODE>), dim3(grid), dim3(256), 0, stream, w, nib, scales, \
-                     nblocks, awq, awq_inv, bpr)
-#define NVE_Q4Q_DT(DT)                                   \
-  if (!awq) NVE_Q4Q(DT, nve::Q4_PLAIN);                  \
-  else if (kquant) NVE_Q4Q(DT, nve::Q4_AWQ_KQUANT);      \
-  else NVE_Q4Q(DT, nve::Q4_AWQ);
-  if (wdt == NVE_DT_F32) {
-    NVE_Q4Q_DT(NVE_DT_F32)
-  } else if (wdt == NVE_DT_BF16) {
-    NVE_Q4Q_DT(NVE_DT_BF16)
-  } else {
-    NVE_Q4Q_DT(NVE_DT_F16)
-  }
-#undef NVE_Q4Q_DT
-#undef NVE_Q4Q
+  if (wdt == NVE_DT_F32)
+    launch_q4_dt<NVE_DT_F32>(w, nblocks, bpr, awq, kquant, nib, scales, awq_inv, stream);
+  else if (wdt == NVE_DT_BF16)
+    launch_q4_dt<NVE_DT_BF16>(w, nblocks, bpr, awq, kquant, nib, scales, awq_inv, stream);
+  else
+    launch_q4_dt<NVE_DT_F16>(w, nblocks, bpr, awq, kquant, nib, scales, awq_inv, stream);
   return hipGetLastError();
 }
 

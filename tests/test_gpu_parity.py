@@ -324,6 +324,32 @@ def test_q4_quantize_awq_device_bit_exact(orc, torch_dev, hk, wdt, kquant):
     assert np.array_equal(down(inv).view(np.uint32), inv_ref.view(np.uint32))
 
 
+@pytest.mark.parametrize("n,k", [(1, 32), (63, 96), (64, 128), (65, 160), (130, 224), (200, 2048)])
+@pytest.mark.parametrize("wdt", ["f32", "bf16"])
+def test_q4_kquant_ragged_bit_exact(orc, torch_dev, hk, n, k, wdt):
+    """The k-quant kernel at the edges of its 64-row x 4-block workgroups (one row, one block, a
+    row and a block past a workgroup, K / 32 not a multiple of 4), against the oracle; and a
+    block holding a NaN or an infinity, for which no candidate has a finite error: scale 0
+    and every code 0 (nibble 8)."""
+    torch = torch_dev
+    rng = np.random.default_rng(n * 100 + k)
+    w = (rng.standard_normal((n, k)) * 0.05).astype(np.float32)
+    wt = torch.from_numpy(w).cuda().to(torch.bfloat16 if wdt == "bf16" else torch.float32)
+    wv = wt.float().cpu().numpy()
+    awq = rng.uniform(0.25, 4.0, k).astype(np.float32)
+    nib, sc, inv = hk.q4_quantize_awq(wt, up(torch, awq), kquant=True)
+    data_ref, inv_ref = orc.q4_from_f32_awq(wv, awq, True)
+    nib_ref, sc_ref = orc.extract_for_gpu(data_ref, n, k)
+    assert np.array_equal(down(nib), nib_ref) and np.array_equal(down(sc), sc_ref)
+    assert np.array_equal(down(inv), inv_ref)
+    for bad in (float("nan"), float("inf"), float("-inf")):
+        wt[n - 1, k - 1] = bad
+        nib2, sc2, _ = hk.q4_quantize_awq(wt, up(torch, awq), kquant=True)
+        assert float(sc2[n - 1, -1]) == 0.0 and bool((nib2[n - 1, -16:] == 0x88).all())
+        nib2[n - 1, -16:], sc2[n - 1, -1] = nib[n - 1, -16:], sc[n - 1, -1]
+        assert torch.equal(nib2, nib) and torch.equal(sc2, sc)
+
+
 def test_q4_quantize_awq_feeds_w4a16_gemv(orc, torch_dev, hk):
     """AWQ end to end: the device-quantized weights and inverse scales through the
     W4A16 GEMV against the float64 dequantized product (bar 2e-3)."""
