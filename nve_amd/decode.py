@@ -262,7 +262,7 @@ class DecodeModel:
         self.token.fill_(int(token))
         check("nve_hip_embed", lib().nve_hip_embed(self.embed.data_ptr(), self.token.data_ptr(),
                                                     self.hidden.data_ptr(), self.shape.hidden, self.shape.vocab,
-                                                    torch.cuda.current_stream().cuda_stream))
+                                                    hk._stream()))
 
     def _advance(self, n: int) -> None:
         if self.length + n > self.max_seq:
@@ -284,13 +284,13 @@ class DecodeModel:
         does not advance the position)."""
         check("nve_hip_layer_forward_decode",
               lib().nve_hip_layer_forward_decode(C.byref(self.cfg), C.byref(self._lw[i]), C.byref(self._io[i]),
-                                                 self.use_w4a8[i], torch.cuda.current_stream().cuda_stream))
+                                                 self.use_w4a8[i], hk._stream()))
 
     def head(self) -> None:
         """Final norm, lm_head, argmax, next-token embedding, position + 1 (enqueued)."""
         check("nve_hip_decode_head",
               lib().nve_hip_decode_head(C.byref(self.cfg), C.byref(self._head), self.lm_head_w4a8,
-                                        torch.cuda.current_stream().cuda_stream))
+                                        hk._stream()))
 
     def capture(self, steps_per_graph: int = 1) -> None:
         """Capture one step as a HIP graph (position and token stay device-side), and,

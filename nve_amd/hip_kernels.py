@@ -26,7 +26,9 @@ _DT = {torch.float16: DT_F16, torch.bfloat16: DT_BF16, torch.float32: DT_F32}
 
 
 def _stream() -> int:
-    return torch.cuda.current_stream().cuda_stream
+    # the current device's current stream as a raw handle: torch.cuda.current_stream() builds a
+    # Stream object for it, 2.5 us of an 8.6 us call (this form: 0.1 us)
+    return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
 
 
 def _dt(t: torch.Tensor) -> int:
@@ -58,7 +60,7 @@ def quantize_f16_q8(x: torch.Tensor) -> tuple[torch.Tensor, torch.Tensor]:
     k = x.numel()
     if k % 32 != 0:
         raise ValueError("quantize_f16_q8: K must be multiple of 32")
-    xf = x.reshape(-1)
+    xf = x if x.is_contiguous() else x.reshape(-1)
     xq = torch.empty(k, dtype=torch.int8, device=x.device)
     sc = torch.empty(k // 32, dtype=torch.float32, device=x.device)
     check("nve_hip_quantize_q8",
@@ -154,7 +156,7 @@ def fused_matvec_w4a16(x, nibbles, scales, awq_scales, n: int, k: int,
     """x[1,K] (fp16/bf16) x W_int4[N,K]^T -> [1,N] (src/cuda_kernels.rs:463-486).
     The output dtype defaults to the activation dtype."""
     out = torch.empty((1, n), dtype=out_dtype or x.dtype, device=x.device)
-    fused_matvec_w4a16_into(x.reshape(-1), nibbles, scales, awq_scales, out, n, k)
+    fused_matvec_w4a16_into(x if x.is_contiguous() else x.reshape(-1), nibbles, scales, awq_scales, out, n, k)
     return out
 
 
@@ -175,7 +177,7 @@ def fused_qkv_matvec_w4a16(x, q_nib, q_sc, q_awq, nq, k_nib, k_sc, k_awq, nk, v_
     """src/cuda_kernels.rs:622-662 -> ([1,Nq], [1,Nk], [1,Nv])."""
     dt = out_dtype or x.dtype
     outs = [torch.empty((1, m), dtype=dt, device=x.device) for m in (nq, nk, nv)]
-    fused_qkv_matvec_w4a16_into(x.reshape(-1), q_nib, q_sc, q_awq, nq, k_nib, k_sc, k_awq, nk, v_nib, v_sc, v_awq,
+    fused_qkv_matvec_w4a16_into(x if x.is_contiguous() else x.reshape(-1), q_nib, q_sc, q_awq, nq, k_nib, k_sc, k_awq, nk, v_nib, v_sc, v_awq,
                                 nv, k_dim, *outs)
     return tuple(outs)
 
