@@ -6,7 +6,7 @@
 // blocks is formed with ws only and multiplied by the row scale at the end).
 //
 // M = 1 runs the one-shot W4A8 GEMV (gemv_w4a8.hip); M >= 2 the LDS-ring int8 MFMA
-// kernel where K % 128 == 0 and N <= 16384, otherwise the staged v_dot4 kernel for M = 2
+// kernel where K % 128 == 0, otherwise (and at M = 2 for N > 16384) the staged v_dot4 kernel for M = 2
 // (where its LDS fits) and the register int8 MFMA kernel.
 // v_dot4 kernel (any M >= 2 under NVE_GEMV_ONESHOT): one wave per output row, lane l owns
 // blocks l, l+64, ...; the nibbles are turned into signed int8 (nib - 8) once per
@@ -396,7 +396,7 @@ __global__ __launch_bounds__(64 * KS) void w4a8_batched_mfma_kernel(int M, const
 
 
 // ---------------------------------------------------------------------------
-// LDS-ring int8 MFMA kernel (M >= 2, K % 128 == 0, N <= 256 * 64).
+// LDS-ring int8 MFMA kernel (M >= 2, K % 128 == 0).
 //
 // Same operand mapping as the kernel above; what changes is how the bytes reach the
 // operand lanes.  The register kernel moves every loaded dword to its operand lane
@@ -419,9 +419,9 @@ __global__ __launch_bounds__(64 * KS) void w4a8_batched_mfma_kernel(int M, const
 // The issue is unconditional (quads past the wave's share are clamped to the last
 // quad), so every quad is the same number of transfers and the waits are exact vmcnt
 // immediates: S quads in flight through the steady loop, an unrolled drain.
-// Workgroups take ceil(N / 256) consecutive rows each (T = ceil(rows / 16) tiles, the
-// last one partly masked), so the grid is at most one workgroup per CU and every CU
-// streams the same number of weight bytes; masked lanes issue no loads.
+// Up to N = 16384 workgroups take ceil(N / 256) consecutive rows each (T = ceil(rows / 16)
+// tiles, the last one partly masked), so the grid is at most one workgroup per CU and every
+// CU streams the same number of weight bytes; masked lanes issue no loads.
 template <int T, int EU, int XS_MODE>
 struct RingLayout {
   static constexpr int MA = EU == 4 ? 2 : 1;  // activation transfers per quad
@@ -648,62 +648,6 @@ static hipError_t launch_mfma(int M, const int8_t* xq, const void* xs, const uin
   return hipGetLastError();
 }
 
-// LDS-ring kernel configuration: 16 waves per workgroup, one quad in flight per wave.
-// Measured on the 8B gate (T = 4) and down (T = 1) shapes at M = 4 / 8 / 16 (us):
-//   16 waves, depth 1:                 gate 9.07 / 9.30 / 10.26   down 9.16 / 9.69 / 11.25
-//   16 waves, depth 2 (down):                                     down 9.21 / 10.48 / 12.21
-//   16 waves, depth 3 (down), 8 waves, depth 3 (gate):
-//                                      gate 9.95 / 10.31 / 10.46  down 9.73 / 10.47 / 12.34
-// Deeper rings do not help (sixteen waves already keep 40-118 KiB per CU in flight).
-template <int T, int EU>
-struct RingCfg {
-  static constexpr int KS = 16;
-  static constexpr int S = 1;
-};
-
-template <int OUT_DT, int XS, int T, int EU>
-static hipError_t launch_ring_t(int M, const int8_t* xq, const void* xs, const uint8_t* nib, const float* ws,
-                                void* out, int N, int K, int rpw, hipStream_t stream) {
-  using C = RingCfg<T, EU>;
-  const int nq = K / 128;
-  if ((nq + C::KS - 1) / C::KS < C::S) return hipErrorNotSupported;
-  const int grid = (N + rpw - 1) / rpw;
-  hipLaunchKernelGGL((nve::w4a8_batched_mfma_lds_kernel<OUT_DT, XS, C::KS, T, EU, C::S>), dim3(grid),
-                     dim3(64 * C::KS), 0, stream, M, xq, xs, nib, ws, out, N, K, rpw);
-  return hipGetLastError();
-}
-
-// hipErrorNotSupported: the shape is outside the ring kernel's range (the caller takes
-// the register kernel).
-template <int OUT_DT, int XS, int EU>
-static hipError_t launch_ring(int M, const int8_t* xq, const void* xs, const uint8_t* nib, const float* ws,
-                              void* out, int N, int K, hipStream_t stream) {
-  constexpr int kCU = 256;
-  if (K % 128 != 0 || N > kCU * 64 || !aligned(ws, 4) || !aligned(xq, 16) || !aligned(nib, 16))
-    return hipErrorNotSupported;
-  const int rpw = N <= 16 * kCU ? 16 : (N + kCU - 1) / kCU;
-  switch ((rpw + 15) / 16) {
-    case 1: return launch_ring_t<OUT_DT, XS, 1, EU>(M, xq, xs, nib, ws, out, N, K, rpw, stream);
-    case 2: return launch_ring_t<OUT_DT, XS, 2, EU>(M, xq, xs, nib, ws, out, N, K, rpw, stream);
-    case 3: return launch_ring_t<OUT_DT, XS, 3, EU>(M, xq, xs, nib, ws, out, N, K, rpw, stream);
-    default: return launch_ring_t<OUT_DT, XS, 4, EU>(M, xq, xs, nib, ws, out, N, K, rpw, stream);
-  }
-}
-
-template <int OUT_DT, int XS>
-static hipError_t launch_mfma_m(int M, const int8_t* xq, const void* xs, const uint8_t* nib, const float* ws,
-                                void* out, int N, int K, hipStream_t stream) {
-  {
-    const hipError_t e = M <= 4   ? launch_ring<OUT_DT, XS, 1>(M, xq, xs, nib, ws, out, N, K, stream)
-                         : M <= 8 ? launch_ring<OUT_DT, XS, 2>(M, xq, xs, nib, ws, out, N, K, stream)
-                                  : launch_ring<OUT_DT, XS, 4>(M, xq, xs, nib, ws, out, N, K, stream);
-    if (e != hipErrorNotSupported) return e;
-  }
-  if (M <= 4) return launch_mfma<OUT_DT, XS, 1>(M, xq, xs, nib, ws, out, N, K, stream);
-  if (M <= 8) return launch_mfma<OUT_DT, XS, 2>(M, xq, xs, nib, ws, out, N, K, stream);
-  return launch_mfma<OUT_DT, XS, 4>(M, xq, xs, nib, ws, out, N, K, stream);
-}
-
 // Staged v_dot4 kernel: the one-row GEMV's tiling (R rows per wave, NJ 64-block chunks
 // per lane, one staging pass), the activation rows in LDS.  It serves M = 2 outside the
 // LDS-ring kernel's range where the two staged rows take at most 40 KB of LDS (8B gate
@@ -720,6 +664,64 @@ static bool staged_fits(int M, int N, int K) {
   s.nseg = 1;
   s.n[0] = N;
   return !choose_w4_tiling(s, K).multi && staged_lds_bytes(M, K) <= 40 * 1024;
+}
+
+// LDS-ring kernel configuration.  N <= 16384 (one workgroup per CU, every CU the same rows):
+// 16 waves per workgroup, one quad in flight per wave.
+// Measured on the 8B gate (T = 4) and down (T = 1) shapes at M = 4 / 8 / 16 (us):
+//   16 waves, depth 1:                 gate 9.07 / 9.30 / 10.26   down 9.16 / 9.69 / 11.25
+//   16 waves, depth 2 (down):                                     down 9.21 / 10.48 / 12.21
+//   16 waves, depth 3 (down), 8 waves, depth 3 (gate):
+//                                      gate 9.95 / 10.31 / 10.46  down 9.73 / 10.47 / 12.34
+// Deeper rings do not help (sixteen waves already keep 40-118 KiB per CU in flight).
+// Larger N (an lm_head): workgroups of 8 waves and 32 rows, two quads in flight per wave,
+// so that two workgroups share a CU and one streams while the other starts or reduces
+// (128256 x 4096, group scales, M = 4 / 8 / 16: 60.9 / 69.4 / 83.3 us; 16 waves of 64 rows, one
+// workgroup per CU: 65.4 / 70.9 / 102.6; 8 waves of 64 rows 66.6 / 71.4 / 81.8; the register
+// kernel 79.1 / 85.7 / 126.5).  With fewer than 16 quads (K < 2048) one quad in flight.
+template <int OUT_DT, int XS, int KS, int T, int EU, int S>
+static hipError_t launch_ring_t(int M, const int8_t* xq, const void* xs, const uint8_t* nib, const float* ws,
+                                void* out, int N, int K, int rpw, hipStream_t stream) {
+  const int grid = (N + rpw - 1) / rpw;
+  hipLaunchKernelGGL((nve::w4a8_batched_mfma_lds_kernel<OUT_DT, XS, KS, T, EU, S>), dim3(grid), dim3(64 * KS), 0,
+                     stream, M, xq, xs, nib, ws, out, N, K, rpw);
+  return hipGetLastError();
+}
+
+// hipErrorNotSupported: the shape is outside the ring kernel's range (the caller takes
+// the register kernel).
+template <int OUT_DT, int XS, int EU>
+static hipError_t launch_ring(int M, const int8_t* xq, const void* xs, const uint8_t* nib, const float* ws,
+                              void* out, int N, int K, hipStream_t stream) {
+  constexpr int kCU = 256;
+  if (K % 128 != 0 || !aligned(ws, 4) || !aligned(xq, 16) || !aligned(nib, 16)) return hipErrorNotSupported;
+  if (N > kCU * 64) {
+    // at M = 2 the staged v_dot4 kernel keeps the shapes it fits (128256 x 4096: 50.7 us against 59.0)
+    if (M == 2 && staged_fits(M, N, K)) return hipErrorNotSupported;
+    if (K < 2048) return launch_ring_t<OUT_DT, XS, 8, 2, EU, 1>(M, xq, xs, nib, ws, out, N, K, 32, stream);
+    return launch_ring_t<OUT_DT, XS, 8, 2, EU, 2>(M, xq, xs, nib, ws, out, N, K, 32, stream);
+  }
+  const int rpw = N <= 16 * kCU ? 16 : (N + kCU - 1) / kCU;
+  switch ((rpw + 15) / 16) {
+    case 1: return launch_ring_t<OUT_DT, XS, 16, 1, EU, 1>(M, xq, xs, nib, ws, out, N, K, rpw, stream);
+    case 2: return launch_ring_t<OUT_DT, XS, 16, 2, EU, 1>(M, xq, xs, nib, ws, out, N, K, rpw, stream);
+    case 3: return launch_ring_t<OUT_DT, XS, 16, 3, EU, 1>(M, xq, xs, nib, ws, out, N, K, rpw, stream);
+    default: return launch_ring_t<OUT_DT, XS, 16, 4, EU, 1>(M, xq, xs, nib, ws, out, N, K, rpw, stream);
+  }
+}
+
+template <int OUT_DT, int XS>
+static hipError_t launch_mfma_m(int M, const int8_t* xq, const void* xs, const uint8_t* nib, const float* ws,
+                                void* out, int N, int K, hipStream_t stream) {
+  {
+    const hipError_t e = M <= 4   ? launch_ring<OUT_DT, XS, 1>(M, xq, xs, nib, ws, out, N, K, stream)
+                         : M <= 8 ? launch_ring<OUT_DT, XS, 2>(M, xq, xs, nib, ws, out, N, K, stream)
+                                  : launch_ring<OUT_DT, XS, 4>(M, xq, xs, nib, ws, out, N, K, stream);
+    if (e != hipErrorNotSupported) return e;
+  }
+  if (M <= 4) return launch_mfma<OUT_DT, XS, 1>(M, xq, xs, nib, ws, out, N, K, stream);
+  if (M <= 8) return launch_mfma<OUT_DT, XS, 2>(M, xq, xs, nib, ws, out, N, K, stream);
+  return launch_mfma<OUT_DT, XS, 4>(M, xq, xs, nib, ws, out, N, K, stream);
 }
 
 template <int OUT_DT, int XS>

@@ -519,6 +519,30 @@ def test_w4a8_batched_mfma_shapes(orc, torch_dev, hk, m, n, k, per_token):
         assert rel_err_floor(y[r], ref) <= TOL_W4A8, r
 
 
+@pytest.mark.parametrize("m,n,k", [(3, 16385, 2048), (8, 16400, 1920), (16, 16417, 128), (5, 20001, 4096),
+                                   (2, 16390, 14464)])
+@pytest.mark.parametrize("per_token", [False, True])
+def test_w4a8_batched_wide_n(orc, torch_dev, hk, m, n, k, per_token):
+    """N > 16384 with K % 128 == 0: the LDS-ring kernel in 32-row workgroups of 8 waves, two
+    quads in flight from 16 quads (K = 2048), one below (15 quads, and a single one, where
+    seven waves have none); a last workgroup of 1, 16 and 1 rows (N = 16385, 16400, 16417);
+    M = 2 where the staged v_dot4 kernel's rows do not fit."""
+    torch = torch_dev
+    print(f"batched wide m={m} n={n} k={k} per_token={per_token}", flush=True)
+    _, _, nib, ws = _problem(orc, n, k, seed=m * 11 + n)
+    x = to_bf16(activations(k, seed=400 + m, m=m))
+    xq, xs = hk.quantize_q8_rows(up(torch, x).to(torch.bfloat16), per_token=per_token)
+    y = down(hk.matvec_w4a8_batched(xq, xs, up(torch, nib), up(torch, ws), n, k, out_dtype=torch.float32))
+    for r in range(m):
+        if per_token:
+            q, s = orc.quantize_q8_rows_bf16(x[r])
+            ref = orc.matvec_w4a8_f64(q[0], orc.bf16_bits_to_f32(s), nib, ws, n, k, xs_mode=1)
+        else:
+            q, s = orc.quantize_q8_group(x[r])
+            ref = orc.matvec_w4a8_f64(q, s, nib, ws, n, k)
+        assert rel_err_floor(y[r], ref) <= TOL_W4A8, r
+
+
 @pytest.mark.parametrize("per_token", [False, True])
 def test_w4a8_batched_graph_replay_matches_eager(orc, torch_dev, hk, per_token):
     """The batched kernels (M = 2 and 5 on the LDS-ring kernel, 16 rows on it at T = 2,
