@@ -22,6 +22,7 @@
 
 #include "common.h"
 #include "lds_ring.h"
+#include "gemm_tile_plan.h"
 #include "w4_launch.h"
 
 namespace nve {
@@ -636,13 +637,6 @@ __global__ __launch_bounds__(256) void split_reduce_kernel(const float* __restri
 namespace nve_host {
 
 constexpr int kGemmSmallM = 16;
-// the register-dequant tile kernel's first M: without K-split partials, and with them
-// (from the first M the ring takes in two launches; workspace path, fp32 out, us: 8B gate
-// M = 80 / 96 / 112 32.5 / 32.9 / 33.4 against 35.8 / 37.7 / 43.8 for the ring launches,
-// 8B down 29.8 / 30.0 / 31.2 against 39.8 / 45.8 / 54.4; at M = 64, one ring launch, 31.5
-// / 28.9 against 24.1 / 28.3)
-constexpr int kGemmTileMinM = 128;
-constexpr int kGemmTileSplitMinM = 65;
 constexpr int kSmallKS = 16;
 
 // K splits of the tiled kernel: split while the tile grid covers fewer than 512
@@ -661,7 +655,7 @@ static int gemm_split(int M, int N, int K, int out_dt) {
 size_t gemm_split_parts_bytes(int M, int N, int K) {
   const int split = gemm_split(M, N, K, NVE_DT_F32);
   const size_t own = split > 1 ? (size_t)split * M * N * sizeof(float) : 0;
-  const size_t tile = M >= kGemmTileSplitMinM ? gemm_tile_parts_bytes(M, N, K) : 0;
+  const size_t tile = M > 64 ? gemm_tile_parts_bytes(M, N, K) : 0;
   return own > tile ? own : tile;
 }
 
@@ -755,6 +749,19 @@ static int ring_rows(bool awq) { return awq ? 32 : 64; }
 // against 76.7 / 88.1 / 109.8 / 116.4 for the tiled kernel; 32-row launches (AWQ) stop
 // winning above 128 rows
 static int ring_chunked_max(bool awq) { return awq ? 128 : 320; }
+// Estimated us of the ring launches of M rows: 2.6 each and, per round of the waves' quads,
+// 0.7 and 0.6 per 16-row weight tile (33 to 64 rows, 6 waves; measured at M = 40: 8B q / gate /
+// down 10.4 / 21 / 28, 2048 x 2048 6.4, 8192 x 2048 8.9, 3072 x 8192 16.2), up to 32 rows (8 waves)
+// 0.6 and 0.58, with AWQ 0.4 and 0.8 (32 rows: q 7.3, gate 17, down 19.3; up to 16 rows 16 waves).
+static double ring_us(int M, int N, int K, bool awq) {
+  const int rows = ring_rows(awq), T = N <= 4096 ? 1 : ((N + 255) / 256 + 15) / 16, nq = K / 128;
+  const int full = M / rows, rest = M % rows;
+  auto one = [&](int m) {
+    if (awq) return 2.6 + (m > 16 ? (nq + 7) / 8 : (nq + 15) / 16) * (0.4 + 0.8 * T);
+    return m > 32 ? 2.6 + (nq + 5) / 6 * (0.7 + 0.6 * T) : 2.6 + (nq + 7) / 8 * (0.6 + 0.58 * T);
+  };
+  return full * one(rows) + (rest ? one(rest) : 0.0);
+}
 static bool ring_fits(int M, int N, int K, bool awq) {
   return M <= ring_rows(awq) && K % 128 == 0 && N <= 16384;
 }
@@ -780,30 +787,27 @@ hipError_t launch_gemm_w4a16_parts(const void* x, int x_dt, int M, const uint8_t
                                    const float* awq, void* out, int out_dt, int N, int K, float* parts,
                                    size_t parts_bytes, hipStream_t s) {
   const bool bf = x_dt == NVE_DT_BF16;
-  // from M = 128 (K % 128 == 0) the 128- / 256-row tile kernel of
-  // gemm_w4a16_tile.hip (with AWQ from M = 65); with K-split partials from M = 65.  Without
-  // them it runs up to the ring launches' range (320 rows, AWQ 128) only where its 128-row
-  // grid has at least 96 workgroups: one workgroup streams all of K, so a narrow grid
-  // leaves the chip idle (fp16 out, us: 8B gate M = 128 / 192 / 256 45.5 / 51.2 / 51.4
-  // against 47.9 / 72.0 / 95.5 for the ring launches; 8B down, 32 column tiles, M = 256:
-  // 133.8 against 120.9 for the ring; above that range the tile kernel beats the 128 x
-  // 128-tile kernel below at both: gate M = 512 81.4 against 124.6, down 143 against
-  // 243).  With the partials a narrow grid is split over K instead.
-  if (M >= kGemmTileSplitMinM && gemm_tile_fits(M, N, K, awq != nullptr)) {
-    const size_t tp = gemm_tile_parts_bytes(M, N, K);
-    const bool split = parts && tp > 0 && parts_bytes >= tp;
-    // (AWQ: from M = 65, where the 32-row ring launches number three or more)
-    const int tile_min = awq ? kGemmTileSplitMinM : kGemmTileMinM;
-    if (split || M > ring_chunked_max(awq != nullptr) || (M >= tile_min && gemm_tile_grid128(M, N) >= 96))
-      return launch_gemm_w4a16_tile(x, x_dt, M, nib, sc, awq, out, out_dt, N, K, split ? parts : nullptr,
-                                    parts_bytes, s);
+  // K % 128 == 0, more than 32 rows: the tile kernel (gemm_w4a16_tile.hip) unless the ring's
+  // launches are estimated faster (narrow outputs up to 64 rows; without a workspace to split K
+  // also some more): workspace path, fp16, us, ring / tile: 8B gate M = 48 21.2 / 19.9, down 27.6 /
+  // 20.5, k_proj 9.3 / 10.1, q_proj 10.6 / 13.5; two ring launches at M = 100: gate 40.6 / 26.2.
+  // The split is planned within the workspace's canonical size, so that it does not vary with
+  // what a caller passes beyond it.
+  const int rr = ring_rows(awq != nullptr);
+  const bool ring_chunks = M <= ring_chunked_max(awq != nullptr) && ring_fits(M < rr ? M : rr, N, K, awq != nullptr);
+  if (M > 32 && gemm_tile_fits(M, N, K, sc)) {
+    const size_t one = (size_t)M * N * sizeof(float), room = gemm_split_parts_bytes(M, N, K);
+    const size_t most = parts && parts_bytes >= room ? room / one : 1;
+    const TilePlan p = plan_gemm_tile(M, N, K, awq != nullptr, most > 1 ? (int)most : 1);
+    // (7% between the two estimates is within their error: the ring, one launch, keeps those)
+    if (!ring_chunks || p.us < 0.93 * ring_us(M, N, K, awq != nullptr))
+      return launch_gemm_w4a16_tile(p, x, x_dt, M, nib, sc, awq, out, out_dt, N, K, parts, s);
   }
   // up to M = 320 (AWQ: 128) where the ring fits: ring launches of up to 64 (AWQ: 32)
   // activation rows each (8B gate, 32-row launches: 27 us at M = 48 and about 58 us at 128, against
   // 45 / 71 us for the tiled kernel); a row's result does not depend on the rows
   // launched with it
-  const int rr = ring_rows(awq != nullptr);
-  if (M > rr && M <= ring_chunked_max(awq != nullptr) && ring_fits(rr, N, K, awq != nullptr)) {
+  if (M > rr && ring_chunks) {
     const size_t osz = out_dt == NVE_DT_F32 ? 4 : 2;
     for (int m0 = 0; m0 < M; m0 += rr) {
       const int mc = M - m0 < rr ? M - m0 : rr;

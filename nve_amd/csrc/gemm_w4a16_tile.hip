@@ -1,4 +1,4 @@
-// gemm_w4a16_tile.hip -- large-M W4A16 prefill GEMM for gfx950: Y[M, N] = X[M, K] W[N, K]^T
+// gemm_w4a16_tile.hip -- W4A16 prefill GEMM for gfx950: Y[M, N] = X[M, K] W[N, K]^T
 // with int4 weights in the reference GPU layout and fp16 / bf16 activations, fp32
 // accumulation.  Same product as the reference's prefill path (GpuWeight::matmul_x,
 // src/gpu_layer.rs:219-237: nve_dequant_w4a16, cuda/nve_kernels.cu:397-433, then a dense
@@ -6,55 +6,65 @@
 // (f32 fma(n, s, -8 s) = (n - 8) s [times awq[k] in f32], then RNE to the activation type)
 // but only in registers.
 //
-// Tile: 256 x 128 outputs per workgroup of 4 waves (2 x 2), 128 x 64 per wave as 4 x 2
-// tiles of v_mfma_f32_32x32x16, or 128 x 128 outputs as 4 waves (1 x 4) of 128 x 32 (4 x 1
-// tiles: each wave dequantizes only its own columns, and a given M has twice the
-// workgroups; the host takes it while that grid is one round); K advances 64 per slice
-// (two Q4 blocks), two slices per barrier (the barrier and each slice's first LDS reads
-// cost about 450 cycles of a 2,700-cycle slice).
-//   * Activation slices: global -> LDS transfers (buffer_load ... lds) one iteration ahead
-//     into two slots of two slices; the A operands are read from LDS (ds_read_b128).
-//   * Weights: the raw blocks (16 B of nibbles and the f32 scale per block row) go to a
-//     three-slot LDS ring two iterations ahead; each wave reads the 8-byte nibble runs of its
-//     64 rows once per slice and forms its B operands in registers (v_cvt_f32_ubyte, fma,
-//     v_cvt_pk), spread between its MFMAs.  With 256-row tiles the two waves sharing a
-//     column block both dequantize it; that VALU work runs beside the matrix pipe, while an LDS copy of the
-//     dequantized weights would cost more LDS bandwidth than the MFMAs leave (measured:
-//     one ds_read_b128 per 32x32x16 MFMA already stretches it from 33 to 47 cycles).
-//   * One barrier per two slices.
-// LDS rows of the activation ring are 128 B (8 chunks of 8 values); chunk c of row r sits
-// at chunk position c ^ ((r >> 1) & 7), so the 16 lanes of each ds_read_b128 phase
-// (rows r .. r + 15 of one chunk) cover all 64 banks.  LDS reads are inline asm with
-// explicit waits: the compiler cannot tell the ring slots apart and would drain every
-// transfer in flight before each access.
-// Workgroup ids are mapped so that each XCD (workgroups are dealt to the 8 XCDs
-// round-robin) runs consecutive tiles of one activation row block: its 2 MiB X slice
-// column stays in that XCD's L2 while the weight tiles stream through.
+// Work split: a workgroup of 8 waves (two per SIMD, so that one wave's dequantization and LDS
+// reads run beside the other's MFMAs) computes a BM x BN tile.  Every wave owns BM x 64
+// outputs (TI x 2 tiles of v_mfma_f32_32x32x16) and an equal share of K: WN waves side by side
+// cover BN, their KG = 8 / WN groups each take one Q4 block (32 of K) of every iteration, and
+// the groups' sums meet in LDS at the end.  So a weight is dequantized once per workgroup and
+// each activation read from LDS feeds two MFMAs; sharing K between the waves instead of
+// columns is what allows both at these tile sizes.
+//   * Global -> LDS transfers only (buffer_load ... lds), in whole 64-byte pieces of a weight
+//     row: nibbles for 128 of K per slot, scales (and AWQ factors) for 512 of K (4-byte scale
+//     transfers per iteration cost as much as the nibbles').  Activations run 3 iterations
+//     ahead (2 with 128 x 128 tiles), nibbles 3-4.
+//   * One barrier per iteration, behind which the MFMAs start at once: their k-step 0 operands
+//     were read and dequantized in the iteration before.
+//   * The transfers and the dequantization are spread over scheduling regions of two MFMAs.
+// What bounds it: the VALU and the MFMAs of an iteration are nearly equal (a wave: 16 MFMAs of
+// 32.5 cycles; 32 weights per lane of about 18 cycles, the conversions v_cvt_f32_ubyte and
+// v_cvt_pk taking 7.5 each) and a full chip clocks lower (0.77 us per 128 x 128 x 128
+// iteration with 32-128 workgroups, 1.04 with 256).  Knockouts, 8B gate M = 512, 128 x 256 tiles,
+// 77 us: no transfers 60, no dequantization 61, neither 51, no MFMAs 48.
+// 8B gate, fp16, us, M = 128 / 256 / 512: 26.9 / 37.6 / 68.9, and q_proj 16.8 / 21.8 / 28.4; a
+// kernel of 4 waves (one per SIMD) with 64 of K per slice, which this one replaced: 32.3 /
+// 46.0 / 73.8 and 22.7 / 24.3 / 34.6.
 #include "common.h"
 #include "lds_ring.h"
+#include "gemm_tile_plan.h"
 #include "w4_launch.h"
 
 namespace nve {
 
-// BM = 256 or 128 activation rows per tile; each wave owns 128 of them and BN / (4 / (BM /
-// 128)) columns: BM = 256 as 2 x 2 waves of 128 x 64, BM = 128 as 1 x 4 waves of 128 x 32
-constexpr int TL_BN = 128, TL_BK = 64;
-__host__ __device__ constexpr int tl_x_bytes(int bm) { return bm * TL_BK * 2; }  // one 64-wide slice
-// raw weights of one slice: 256 blocks x (16 B nibbles, 4 B scale) = 5 KiB, and with AWQ the
-// slice's 64 factors (256 B) after them
-__host__ __device__ constexpr int tl_r_bytes(bool awq) { return TL_BN * 2 * 20 + (awq ? 256 : 0); }
-// An iteration (one barrier) covers two slices: two activation slots of two slices each,
-// three raw weight slots of two slices each (BM = 256: 158 KiB, 159.5 with AWQ; 128: 94 KiB)
-__host__ __device__ constexpr int tl_r0(int bm) { return 2 * 2 * tl_x_bytes(bm); }
-__host__ __device__ constexpr int tl_lds_bytes(int bm, bool awq) { return tl_r0(bm) + 3 * 2 * tl_r_bytes(awq); }
+constexpr int kTlWaves = 8;
 
 typedef _Float16 tl_h8_t __attribute__((ext_vector_type(8)));
 typedef __bf16 tl_b8_t __attribute__((ext_vector_type(8)));
 typedef float tl_f16x_t __attribute__((ext_vector_type(16)));
+typedef float tl_f4_t __attribute__((ext_vector_type(4)));
 typedef float tl_f2_t __attribute__((ext_vector_type(2)));
 typedef _Float16 tl_h2_t __attribute__((ext_vector_type(2)));
 typedef __bf16 tl_b2_t __attribute__((ext_vector_type(2)));
-typedef unsigned int tl_u2_t __attribute__((ext_vector_type(2)));
+
+// One workgroup: a BM x BN tile by 8 waves, WN of them side by side (64 columns each) in KG =
+// 8 / WN groups that split K.  LDS: 4 activation slots (BM rows x KG blocks of 64 B), 3 nibble
+// slots (BN rows x 4 blocks of 16 B), 2 scale slots (BN rows x 16 blocks), with AWQ the
+// factors of the same 16 blocks; the final exchange of the K groups' sums reuses it.
+template <int TI, int WN, bool AWQ>
+struct TileCfg {
+  static constexpr int KG = kTlWaves / WN;
+  static constexpr int BM = 32 * TI, BN = 64 * WN;
+  static constexpr int IK = 32 * KG;           // K of one iteration
+  static constexpr int NIT = 128 / IK;         // iterations per nibble slot
+  static constexpr int SIT = 512 / IK;         // iterations per scale slot
+  static constexpr int X = BM * 64 * KG, NIB = BN * 64, SC = BN * 64, AW = AWQ ? 2048 : 0;
+  // 128 x 128 tiles leave room for 3 activation slots (one iteration ahead less)
+  static constexpr int XS = TI == 4 && WN == 2 ? 3 : 4;
+  static constexpr int N0 = XS * X, S0 = N0 + 3 * NIB, A0 = S0 + 2 * SC;
+  static constexpr int RING = A0 + 2 * AW;
+  static constexpr int RED = kTlWaves * TI * 16 * 256;  // half of every wave's sums
+  static constexpr int BYTES = RING > RED ? RING : RED;
+  static_assert(BYTES <= 160 * 1024, "LDS");
+};
 
 template <bool BF16>
 __device__ __forceinline__ tl_f16x_t tl_mfma(u32x4_t a, u32x4_t b, tl_f16x_t c) {
@@ -65,25 +75,6 @@ __device__ __forceinline__ tl_f16x_t tl_mfma(u32x4_t a, u32x4_t b, tl_f16x_t c) 
                                                 0, 0);
 }
 
-template <int OFF>
-__device__ __forceinline__ u32x4_t tl_ds_read128(uint32_t a) {
-  u32x4_t v;
-  asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(v) : "v"(a), "i"(OFF));
-  return v;
-}
-template <int OFF>
-__device__ __forceinline__ tl_u2_t tl_ds_read64(uint32_t a) {
-  tl_u2_t v;
-  asm volatile("ds_read_b64 %0, %1 offset:%2" : "=v"(v) : "v"(a), "i"(OFF));
-  return v;
-}
-template <int OFF>
-__device__ __forceinline__ uint32_t tl_ds_read32(uint32_t a) {
-  uint32_t v;
-  asm volatile("ds_read_b32 %0, %1 offset:%2" : "=v"(v) : "v"(a), "i"(OFF));
-  return v;
-}
-
 template <bool BF16>
 __device__ __forceinline__ uint32_t tl_pack2(float a, float b) {
   // each value is an f32 first (the fma's rounding), then one v_cvt_pk_{f16,bf16}_f32
@@ -92,412 +83,452 @@ __device__ __forceinline__ uint32_t tl_pack2(float a, float b) {
   if (BF16) return __builtin_bit_cast(uint32_t, __builtin_convertvector((tl_f2_t){a, b}, tl_b2_t));
   return __builtin_bit_cast(uint32_t, __builtin_convertvector((tl_f2_t){a, b}, tl_h2_t));
 }
-// The reference dequant of 8 nibbles -- one per byte of lo (values 0..3) and hi (values
-// 4..7), already masked -- [times the AWQ factors a0 (values 0..3) and a1 (4..7), each an
-// f32 product of the f32 dequantized value as the reference forms it,] rounded to the
-// activation type and packed in k order.
+// The reference dequant of 4 nibbles, one per byte of d (already masked) [times the AWQ
+// factors a, each an f32 product of the f32 dequantized value as the reference forms it,]
+// rounded to the activation type and packed in k order.
 template <bool BF16, bool AWQ>
-__device__ __forceinline__ u32x4_t tl_dequant8(uint32_t lo, uint32_t hi, float s, float s8, const u32x4_t& a0,
-                                               const u32x4_t& a1) {
-  // the masked dwords are opaque to the compiler, so each byte goes through one
+__device__ __forceinline__ u32x2_t tl_dequant4(uint32_t d, float s, float s8, const tl_f4_t& a) {
+  // the masked dword is opaque to the compiler, so each byte goes through one
   // v_cvt_f32_ubyte{0..3} (instead of a bit-field extract and a conversion)
-  asm("" : "+v"(lo), "+v"(hi));
-  float v[8];
+  asm("" : "+v"(d));
+  float v[4];
 #pragma unroll
   for (int t = 0; t < 4; ++t) {
-    v[t] = fmaf((float)((lo >> (8 * t)) & 0xffu), s, s8);
-    v[4 + t] = fmaf((float)((hi >> (8 * t)) & 0xffu), s, s8);
+    v[t] = fmaf((float)((d >> (8 * t)) & 0xffu), s, s8);
+    if constexpr (AWQ) v[t] *= a[t];
   }
-  if constexpr (AWQ) {
-    const uint32_t f[8] = {a0.x, a0.y, a0.z, a0.w, a1.x, a1.y, a1.z, a1.w};
-#pragma unroll
-    for (int e = 0; e < 8; ++e) v[e] *= __builtin_bit_cast(float, f[e]);
-  }
-  u32x4_t r;
+  u32x2_t r;
   r.x = tl_pack2<BF16>(v[0], v[1]);
   r.y = tl_pack2<BF16>(v[2], v[3]);
-  r.z = tl_pack2<BF16>(v[4], v[5]);
-  r.w = tl_pack2<BF16>(v[6], v[7]);
   return r;
 }
 
-// SPLIT: blockIdx.y = z takes slices z ks .. z ks + ks - 1 of K (ks even) and stores its
-// fp32 partial tile to out + z M N (tl_reduce_kernel adds the partials in order).
-// AWQ: the weights are multiplied by awq[k] after the dequant, as the reference does.
-template <bool BF16, bool AWQ, int OUT_DT, int BM, bool SPLIT>
-__global__ __launch_bounds__(256, 1) void gemm_w4a16_tile_kernel(const uint16_t* __restrict__ x,
-                                                                 const uint8_t* __restrict__ nib,
-                                                                 const float* __restrict__ sc,
-                                                                 const float* __restrict__ awq, void* __restrict__ out,
-                                                                 int M, int N, int K, int n_tiles, int ks) {
+typedef __attribute__((address_space(3))) char tl_lds_t;
+
+// What a wave holds of one iteration's weights: per column tile the 8 nibble bytes of its
+// k-run and the block scale, and with AWQ the 8 factors of each of the two k-steps.
+template <bool AWQ>
+struct TileRaw {
+  u32x2_t q[2];
+  float s[2];
+  tl_f4_t aw[AWQ ? 4 : 1];
+};
+
+// Quarter c of a k-step's two B operands: values 4 (c % 2) .. + 3 of column tile c / 2.
+template <bool BF16, bool AWQ, int KK>
+__device__ __forceinline__ void tl_b_quarter(u32x4_t (&f)[2], const TileRaw<AWQ>& w, int c) {
+  const int j = c >> 1;
+  const uint32_t q = (c & 1) ? w.q[j].y : w.q[j].x;
+  const u32x2_t v = tl_dequant4<BF16, AWQ>(KK ? (q >> 4) & 0x0F0F0F0Fu : q & 0x0F0F0F0Fu, w.s[j], -8.0f * w.s[j],
+                                           w.aw[AWQ ? 2 * KK + (c & 1) : 0]);
+  if (c & 1) {
+    f[j].z = v.x;
+    f[j].w = v.y;
+  } else {
+    f[j].x = v.x;
+    f[j].y = v.y;
+  }
+}
+
+// SPLIT: blockIdx.y = z takes iterations z ks .. z ks + ks - 1 of K and stores its fp32
+// partial tile to out + z M N (tl_reduce_kernel adds the partials in order).
+template <bool BF16, bool AWQ, int OUT_DT, int TI, int WN, bool SPLIT>
+__global__ __launch_bounds__(64 * kTlWaves) __attribute__((amdgpu_waves_per_eu(2, 2))) void gemm_w4a16_tile_kernel(
+    const uint16_t* __restrict__ x, const uint8_t* __restrict__ nib, const float* __restrict__ sc,
+    const float* __restrict__ awq, void* __restrict__ out, int M, int N, int K, int n_tiles, int ks) {
   static_assert(!SPLIT || OUT_DT == NVE_DT_F32, "split partials are fp32");
-  extern __shared__ __align__(16) char tl_lds[];
-  static_assert(BM == 256 || BM == 128, "row tile");
-  constexpr int WM = BM / 128;    // waves along M (each 128 rows)
-  constexpr int TJ = WM;          // 32-column MFMA tiles per wave: BN / (4 / WM) / 32
-  constexpr int NX = BM / 32;     // activation transfers (1 KiB) per wave and slice
-  constexpr int TL_X = tl_x_bytes(BM), TL_R0 = tl_r0(BM), TL_R = tl_r_bytes(AWQ);
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int wm = wave / (4 / WM), wn = wave % (4 / WM);
+#ifdef __HIP_DEVICE_COMPILE__  // (the host pass has no use for the body and cannot lower its LDS accesses)
+  extern __shared__ __align__(16) char tl_smem[];
+  using C = TileCfg<TI, WN, AWQ>;
+  constexpr int KG = C::KG, BM = C::BM, BN = C::BN;
+  static_assert(KG == 2 || KG == 4, "K groups");
+  constexpr int XT = 2 * TI * KG;                   // activation transfers (1 KiB) of an iteration
+  constexpr int NX = (XT + kTlWaves - 1) / kTlWaves;  // per wave, at most
+  constexpr int NXMIN = XT / kTlWaves;                // and at least
+  constexpr int NS = BN / 16 / kTlWaves;              // scale transfers per wave and slot
+  constexpr int RS = 64 * KG, NCH = 4 * KG;  // LDS row bytes / 16-byte chunks of an activation row
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int g = wave / WN, wn = wave % WN;
 
   // XCD-grouped tile order: block b runs on XCD b % 8; the blocks of one XCD take
   // consecutive linear tiles (row block major)
   const int total = gridDim.x, b = blockIdx.x, xcd = b & 7;
   const int per = total >> 3, extra = total & 7;
   const int lin = xcd * per + min(xcd, extra) + (b >> 3);
-  const int m0 = (lin / n_tiles) * BM, n0 = (lin % n_tiles) * TL_BN;
-  // this workgroup's slices: t0 .. t0 + T - 1
+  const int m0 = (lin / n_tiles) * BM, n0 = (lin % n_tiles) * BN;
+  // this workgroup's iterations: t0 .. t0 + T - 1 (t0 a multiple of the nibble slot's)
   const int t0 = SPLIT ? (int)blockIdx.y * ks : 0;
-  const int T = SPLIT ? min(K / TL_BK - t0, ks) : K / TL_BK;
-  const uint32_t lds0 = lds_addr(tl_lds);
+  const int T = SPLIT ? min(K / C::IK - t0, ks) : K / C::IK;
 
-  // buffer resources (raw buffers, 32-bit offsets: the host routes M K >= 2^30
-  // elsewhere): transfers take the per-lane offset in a VGPR, the slice offset in an SGPR
-  const __amdgpu_buffer_rsrc_t xr = __builtin_amdgcn_make_buffer_rsrc((void*)x, (short)0, 0x7fffffff, 0x00020000);
-  const __amdgpu_buffer_rsrc_t nr = __builtin_amdgcn_make_buffer_rsrc((void*)nib, (short)0, 0x7fffffff, 0x00020000);
-  const __amdgpu_buffer_rsrc_t sr = __builtin_amdgcn_make_buffer_rsrc((void*)sc, (short)0, 0x7fffffff, 0x00020000);
+  // buffer resources (raw buffers, 32-bit offsets: the host routes larger operands elsewhere;
+  // a read past the end of the scales or factors -- the last slot of a K that is no multiple
+  // of 512 -- returns 0): per-lane offset in a VGPR, the iteration's in an SGPR
+  const __amdgpu_buffer_rsrc_t xr = __builtin_amdgcn_make_buffer_rsrc((void*)x, (short)0, 2 * M * K, 0x00020000);
+  const __amdgpu_buffer_rsrc_t nr = __builtin_amdgcn_make_buffer_rsrc((void*)nib, (short)0, N * (K / 2), 0x00020000);
+  const __amdgpu_buffer_rsrc_t sr = __builtin_amdgcn_make_buffer_rsrc((void*)sc, (short)0, N * (K / 8), 0x00020000);
   const __amdgpu_buffer_rsrc_t ar =
-      __builtin_amdgcn_make_buffer_rsrc((void*)(AWQ ? awq : sc), (short)0, 0x7fffffff, 0x00020000);
-  // activation transfers: instruction i of wave w fills tile rows (BM / 4) w + 8 i .. + 7
-  // (1 KiB); lane l writes row (BM / 4) w + 8 i + l / 8 at chunk position l % 8, i.e. global
-  // chunk (l % 8) ^ ((row >> 1) & 7)
-  uint32_t xoff[8];
+      __builtin_amdgcn_make_buffer_rsrc((void*)(AWQ ? awq : sc), (short)0, AWQ ? 4 * K : 0, 0x00020000);
+  // activation transfers: instruction i fills 1024 / RS tile rows; lane l writes row l / NCH of
+  // them at chunk position l % NCH, i.e. global chunk position ^ swizzle(row)
+  auto swz = [](int r) { return KG == 4 ? (r & 15) : ((r >> 1) & 7); };
+  uint32_t xoff[NX];
 #pragma unroll
   for (int i = 0; i < NX; ++i) {
-    const int r = (BM / 4) * wave + 8 * i + (lane >> 3);
-    const int c = (lane & 7) ^ ((r >> 1) & 7);
+    const int r = (kTlWaves * i + wave) * (1024 / RS) + lane / NCH;
+    const int c = (lane % NCH) ^ swz(r);
     xoff[i] = ((uint32_t)min(m0 + r, M - 1) * (uint32_t)K + 8u * c) * 2u;
   }
-  // raw weights of a slice: block q = tid (tile row q / 2, block q % 2 of the slice): its
-  // 16 B of nibbles go to R + 16 q, its scale to R + 4096 + 4 q
-  const int rrow = min(n0 + (tid >> 1), N - 1);
-  const uint32_t noff = (uint32_t)rrow * (uint32_t)(K / 2) + 16u * (tid & 1);
-  const uint32_t soff = ((uint32_t)rrow * (uint32_t)(K / 32) + (tid & 1)) * 4u;
+  // weight transfers (1 KiB: 16 rows x 64 B): lane l carries row 16 i + l / 4 of the tile, 16-byte
+  // position l % 4, which holds chunk (position - row / 4) % 4 of the slot's 64 bytes (so that the
+  // rows read together fall on different banks)
+  constexpr int NW = BN / 16 / kTlWaves;  // row groups per wave
+  uint32_t noff[NW], soff[NW];
+#pragma unroll
+  for (int i = 0; i < NW; ++i) {
+    const int r = 16 * (kTlWaves * i + wave) + (lane >> 2);
+    const uint32_t rg = (uint32_t)min(n0 + r, N - 1), c = ((lane & 3) - (r >> 2)) & 3;
+    noff[i] = rg * (uint32_t)(K / 2) + 16u * c;
+    soff[i] = rg * (uint32_t)(K / 8) + 16u * c;
+  }
 
-  // A fragments: rows 128 wm + 32 i + l % 32 (tile i at +4096 i); chunk position of step
-  // kk: (2 kk + l / 32) ^ (((l % 32) >> 1) & 7)
-  const int fr = lane & 31, fsw = (fr >> 1) & 7, fhi = lane >> 5;
-  const uint32_t arow = (128 * wm + fr) * 128;
-  uint32_t koff[4];
-#pragma unroll
-  for (int kk = 0; kk < 4; ++kk) koff[kk] = ((2 * kk + fhi) ^ fsw) * 16;
-  // B operands: lane l of step kk takes row 32 (TJ wn + j) + l % 32, values 16 kk + 8 (l / 32)
-  // .. + 7 of the slice = block kk / 2, nibble bytes 8 (l / 32) .. + 7, low nibbles for even
-  // kk and high for odd: one 8-byte read per (j, block) serves two steps
-  const uint32_t bq = (uint32_t)(2 * (32 * TJ * wn + fr)) * 16 + 8 * fhi;  // + j * 1024 + block * 16
-  const uint32_t bs = 4096 + (uint32_t)(2 * (32 * TJ * wn + fr)) * 4;      // + j * 256 + block * 4
+  // A fragments: rows 32 i + l % 32, chunk 4 g + 2 kk + l / 32 of the row
+  const int fr = lane & 31, fhi = lane >> 5;
+  const uint32_t a0 = fr * RS + 16 * ((4 * g + fhi) ^ swz(fr)), a1 = fr * RS + 16 * ((4 * g + 2 + fhi) ^ swz(fr));
+  // B operands: column tile j of the wave covers rows 64 wn + 32 j + l % 32; nibble bytes
+  // 8 (l / 32) .. + 7 of the group's block: low nibbles are k-step 0's values, high ones k-step 1's
+  const int wrow = 64 * wn + fr, wq = wrow >> 2;
+  const uint32_t bq = wrow * 64 + 16 * ((g + wq) & 3) + 8 * fhi;
+  constexpr int TSTEP = 32 * 64;  // column tile 1
 
-  tl_f16x_t acc[4][2];
+  tl_f16x_t acc[2 * TI];  // [2 i + j]
 #pragma unroll
-  for (int i = 0; i < 4; ++i)
-#pragma unroll
-    for (int j = 0; j < 2; ++j) acc[i][j] = tl_f16x_t{};
+  for (int i = 0; i < 2 * TI; ++i) acc[i] = tl_f16x_t{};
 
-  // transfers of slice t (clamped to the last slice: the ones past the end re-read it,
-  // which keeps every iteration's transfer count equal)
-  auto issue_raw = [&](int t, int rslot) {
-    const int tc = t0 + min(t, T - 1);
-    char* const rb = tl_lds + TL_R0 + (2 * rslot + (t & 1)) * TL_R;
-    __builtin_amdgcn_raw_ptr_buffer_load_lds(nr, (lds_void_t*)(rb + wave * 1024), 16, noff, tc * 32, 0, 0);
-    __builtin_amdgcn_raw_ptr_buffer_load_lds(sr, (lds_void_t*)(rb + 4096 + wave * 256), 4, soff, tc * 8, 0, 0);
-    // the slice's 64 AWQ factors, one per lane of wave 0 (the others' transfer counts are
-    // unchanged; wave 0 waits for two more per iteration)
-    if (AWQ && wave == 0)
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(ar, (lds_void_t*)(rb + 5120), 4, 4u * lane, tc * 256, 0, 0);
+  tl_lds_t* const lds = (tl_lds_t*)tl_smem;
+  // transfers (iterations and slots past the end re-read the last ones, which keeps every
+  // iteration's transfer count equal)
+  auto issue_x = [&](int e, tl_lds_t* d, int t) __attribute__((always_inline)) {
+    if (XT % kTlWaves == 0 || kTlWaves * e + wave < XT)
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(xr, (lds_void_t*)(d + (kTlWaves * e + wave) * 1024), 16, xoff[e],
+                                               (t0 + min(t, T - 1)) * (64 * KG), 0, 0);
   };
-  // activation transfers i0 .. i1 - 1 of slice t
-  auto issue_x_part = [&](int t, int xslot, int i0, int i1) {
-    const int ko = (t0 + min(t, T - 1)) * (TL_BK * 2);
-    char* const base = tl_lds + (2 * xslot + (t & 1)) * TL_X + wave * (BM / 4) * 128;
+  const int pmax = (T - 1) / C::NIT, p0 = t0 / C::NIT;
+  auto issue_nib = [&](int i, tl_lds_t* d, int p) __attribute__((always_inline)) {
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(nr, (lds_void_t*)(d + (kTlWaves * i + wave) * 1024), 16, noff[i],
+                                             (p0 + min(p, pmax)) * 64, 0, 0);
+  };
+  const int smax = (T - 1) / C::SIT;
+  auto issue_sc = [&](tl_lds_t* d, tl_lds_t* da, int p) __attribute__((always_inline)) {
+    const int pc = min(p, smax);
 #pragma unroll
-    for (int i = i0; i < i1; ++i)
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(xr, (lds_void_t*)(base + i * 1024), 16, xoff[i], ko, 0, 0);
+    for (int i = 0; i < NS; ++i)
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(sr, (lds_void_t*)(d + (kTlWaves * i + wave) * 1024), 16, soff[i],
+                                               t0 * (4 * KG) + pc * 64, 0, 0);
+    if (AWQ && wave < 2)
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(ar, (lds_void_t*)(da + wave * 1024), 16, wave * 1024 + lane * 16,
+                                               t0 * (128 * KG) + pc * 2048, 0, 0);
   };
-  auto issue_x = [&](int t, int xslot) { issue_x_part(t, xslot, 0, NX); };  // slice t into its half of xslot
-  auto rd_a = [&](uint32_t xa, int kk, u32x4_t (&fa)[4]) {
-    const uint32_t a = xa + arow + koff[kk];
-    fa[0] = tl_ds_read128<0>(a);
-    fa[1] = tl_ds_read128<4096>(a);
-    fa[2] = tl_ds_read128<8192>(a);
-    fa[3] = tl_ds_read128<12288>(a);
-  };
-  // B operand of step kk for one column tile from its raw run q (block kk / 2)
-  auto b_operand = [&](const tl_u2_t& q, float s, int kk, const u32x4_t& a0, const u32x4_t& a1) {
-    const uint32_t lo = (kk & 1) ? (q.x >> 4) & 0x0F0F0F0Fu : q.x & 0x0F0F0F0Fu;
-    const uint32_t hi = (kk & 1) ? (q.y >> 4) & 0x0F0F0F0Fu : q.y & 0x0F0F0F0Fu;
-    return tl_dequant8<BF16, AWQ>(lo, hi, s, -8.0f * s, a0, a1);
-  };
-  // AWQ factors of the lane's 8 values of step kk: slice values 16 kk + 8 (l / 32) .. + 7
-  const uint32_t aoff = 5120 + 32 * fhi;  // + 64 kk
-  // the MFMAs of one slice (activations at LDS xa, raw weights at rb): A fragments of step
-  // kk + 1 are read and B operands of step kk + 1 formed while step kk multiplies (each
-  // MFMA followed by VALU work); iss(kk) issues transfers of later slices beside the
-  // MFMAs of step kk: issued back to back after the barrier, the four waves' transfers
-  // held the address pipeline for about 500 cycles with no matrix work in flight
-  auto mma = [&](uint32_t xa, uint32_t rb, auto&& iss) {
-    tl_u2_t q[2][2];  // [j][block]
-    uint32_t sbits[2][2];
-    u32x4_t fa[4];
-    u32x4_t aw[4][2] = {};  // AWQ factors of steps 0..3 (unused without AWQ)
+  // the raw weights of iteration u (its nibble slot nb, scale slot sb, factors ab)
+  auto read_raw = [&](TileRaw<AWQ>& w, const tl_lds_t* nb, const tl_lds_t* sb, const tl_lds_t* ab, int u)
+      __attribute__((always_inline)) {
+    const uint32_t q = C::NIT == 2 ? bq ^ ((u & 1) << 5) : bq;  // block 2 (u % 2) + g of the slot
+    const int blk = (u % C::SIT) * KG + g;                      // of the scale slot's 16
+    const uint32_t s = wrow * 64 + 16 * (((blk >> 2) + wq) & 3) + 4 * (blk & 3);
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      w.q[j] = *(const __attribute__((address_space(3))) u32x2_t*)(nb + q + j * TSTEP);
+      w.s[j] = *(const __attribute__((address_space(3))) float*)(sb + s + j * TSTEP);
+    }
     if constexpr (AWQ) {
-      aw[0][0] = tl_ds_read128<0>(rb + aoff);
-      aw[0][1] = tl_ds_read128<16>(rb + aoff);
-      aw[1][0] = tl_ds_read128<64>(rb + aoff);
-      aw[1][1] = tl_ds_read128<80>(rb + aoff);
-      aw[2][0] = tl_ds_read128<128>(rb + aoff);
-      aw[2][1] = tl_ds_read128<144>(rb + aoff);
-      aw[3][0] = tl_ds_read128<192>(rb + aoff);
-      aw[3][1] = tl_ds_read128<208>(rb + aoff);
-    }
-    q[0][0] = tl_ds_read64<0>(rb + bq);
-    q[0][1] = tl_ds_read64<16>(rb + bq);
-    sbits[0][0] = tl_ds_read32<0>(rb + bs);
-    sbits[0][1] = tl_ds_read32<4>(rb + bs);
-    if (TJ == 2) {
-      q[1][0] = tl_ds_read64<1024>(rb + bq);
-      q[1][1] = tl_ds_read64<1040>(rb + bq);
-      sbits[1][0] = tl_ds_read32<256>(rb + bs);
-      sbits[1][1] = tl_ds_read32<260>(rb + bs);
-    }
-    rd_a(xa, 0, fa);
-    lgkm_wait();
-#pragma unroll
-    for (int j = 0; j < TJ; ++j)
-#pragma unroll
-      for (int h = 0; h < 2; ++h) {
-        tie(q[j][h]);
-        tie(sbits[j][h]);
-      }
-    if constexpr (AWQ) {
-#pragma unroll
-      for (int kk = 0; kk < 4; ++kk) {
-        tie(aw[kk][0]);
-        tie(aw[kk][1]);
-      }
-    }
-    float s[2][2];
-#pragma unroll
-    for (int j = 0; j < TJ; ++j)
-#pragma unroll
-      for (int h = 0; h < 2; ++h) s[j][h] = __builtin_bit_cast(float, sbits[j][h]);
-    u32x4_t fb[2];
-#pragma unroll
-    for (int j = 0; j < TJ; ++j) fb[j] = b_operand(q[j][0], s[j][0], 0, aw[0][0], aw[0][1]);
-#pragma unroll
-    for (int kk = 0; kk < 4; ++kk) {
-      if (kk > 0) lgkm_wait();
-#pragma unroll
-      for (int i = 0; i < 4; ++i) tie(fa[i]);
-      u32x4_t ca[4], cb[2];
-#pragma unroll
-      for (int i = 0; i < 4; ++i) ca[i] = fa[i];
-#pragma unroll
-      for (int j = 0; j < TJ; ++j) cb[j] = fb[j];
-      if (kk < 3) rd_a(xa, kk + 1, fa);
-      iss(kk);
-      // one scheduling region: the 8 MFMAs of step kk with the next step's B operands
-      // formed between them
-      if (kk < 3) {
-#pragma unroll
-        for (int j = 0; j < TJ; ++j)
-          fb[j] = b_operand(q[j][(kk + 1) >> 1], s[j][(kk + 1) >> 1], kk + 1, aw[kk + 1][0], aw[kk + 1][1]);
-      }
 #pragma unroll
       for (int i = 0; i < 4; ++i)
+        w.aw[i] = *(const __attribute__((address_space(3))) tl_f4_t*)(ab + blk * 128 + 32 * fhi + (i & 1) * 16 +
+                                                                      (i >> 1) * 64);
+    }
+  };
+  auto read_a = [&](u32x4_t (&f)[TI], const tl_lds_t* xs, uint32_t a) __attribute__((always_inline)) {
 #pragma unroll
-        for (int j = 0; j < TJ; ++j) acc[i][j] = tl_mfma<BF16>(ca[i], cb[j], acc[i][j]);
-      if (kk < 3) {
+    for (int i = 0; i < TI; ++i) f[i] = *(const __attribute__((address_space(3))) u32x4_t*)(xs + a + i * 32 * RS);
+  };
+
+  // Pipeline: iteration u issues the activations of u + 3, its share of a nibble slot 3 (KG = 4)
+  // or 2 (KG = 2: two iterations each) ahead and, as the first of a scale slot, the next one;
+  // it reads the k-step 0 activations and the raw weights of u + 1 and forms that step's
+  // operands, so that the next iteration's MFMAs start right behind its barrier.
+  constexpr int PD = C::NIT == 2 ? 2 : 3;  // nibble slots ahead
+  issue_sc(lds + C::S0, lds + C::A0, 0);
 #pragma unroll
-        for (int m = 0; m < 4 * TJ; ++m) {
-          __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-          __builtin_amdgcn_sched_group_barrier(0x002, 6, 0);
+  for (int p = 0; p < PD; ++p)
+#pragma unroll
+    for (int i = 0; i < NW; ++i) issue_nib(i, lds + C::N0 + p * C::NIB, p);
+#pragma unroll
+  for (int i = 0; i < C::XS - 1; ++i)
+#pragma unroll
+    for (int e = 0; e < NX; ++e) issue_x(e, lds + i * C::X, i);
+  u32x4_t fa[TI], fb[2];
+  TileRaw<AWQ> cur;
+  wait_vmcnt<C::XS == 4 ? NXMIN : 0>();
+  lds_barrier();
+  // (the slots read and those the transfers fill are different objects to the compiler
+  // (restrict), so it adds no waits of its own for the transfers)
+  auto first = [&](const tl_lds_t* __restrict__ r, tl_lds_t* __restrict__ none) __attribute__((always_inline)) {
+    read_a(fa, r, a0);
+    read_raw(cur, r + C::N0, r + C::S0, r + C::A0, 0);
+  };
+  first(lds, lds + C::X);
+#pragma unroll
+  for (int c = 0; c < 4; ++c) tl_b_quarter<BF16, AWQ, 0>(fb, cur, c);
+
+  auto iter = [&](const tl_lds_t* __restrict__ rd, tl_lds_t* __restrict__ wr, int x0, int x1, int n1, int s1, int xd,
+                  int nd, int sd, int u) __attribute__((always_inline)) {
+    u32x4_t fa1[TI], fb1[2];
+    TileRaw<AWQ> nxt;
+    read_a(fa1, rd + x0 * C::X, a1);
+    read_raw(nxt, rd + C::N0 + n1 * C::NIB, rd + C::S0 + s1 * C::SC, rd + C::A0 + s1 * C::AW, u + 1);
+    // one scheduling region per two MFMAs, each with its share of the transfers and of the
+    // next k-step's dequantization: left in one group the transfers of the eight waves
+    // hold the address pipeline while no MFMA runs
+    auto extra = [&](int r) __attribute__((always_inline)) {
+#pragma unroll
+      for (int e = 0; e < NX; ++e)
+        if (r == e) issue_x(e, wr + xd * C::X, u + C::XS - 1);
+      if (r == TI) {
+        if constexpr (C::NIT == 1) {
+          issue_nib(0, wr + C::N0 + nd * C::NIB, u + 3);
+        } else if ((u & 1) == 0) {
+          issue_nib(0, wr + C::N0 + nd * C::NIB, (u >> 1) + 2);
+        } else {
+          issue_nib(NW - 1, wr + C::N0 + nd * C::NIB, (u >> 1) + 2);
         }
+      }
+      if (r == TI + 1 && u % C::SIT == 0) issue_sc(wr + C::S0 + sd * C::SC, wr + C::A0 + sd * C::AW, u / C::SIT + 1);
+    };
+#pragma unroll
+    for (int i = 0; i < TI; ++i) {
+#pragma unroll
+      for (int j = 0; j < 2; ++j) acc[2 * i + j] = tl_mfma<BF16>(fa[i], fb[j], acc[2 * i + j]);
+      extra(i);
+#pragma unroll
+      for (int c = 4 * i / TI; c < 4 * (i + 1) / TI; ++c) tl_b_quarter<BF16, AWQ, 1>(fb1, cur, c);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    read_a(fa, rd + x1 * C::X, a0);
+#pragma unroll
+    for (int i = 0; i < TI; ++i) {
+#pragma unroll
+      for (int j = 0; j < 2; ++j) acc[2 * i + j] = tl_mfma<BF16>(fa1[i], fb1[j], acc[2 * i + j]);
+      extra(TI + i);
+#pragma unroll
+      for (int c = 4 * i / TI; c < 4 * (i + 1) / TI; ++c) tl_b_quarter<BF16, AWQ, 0>(fb, nxt, c);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    cur = nxt;
+  };
+  static_assert(NX <= TI, "one activation transfer per region");
+  int xs = 0, ns = 0;  // slots of iteration u's activations and nibbles
+  for (int u = 0; u < T; ++u) {
+    // all but the transfers of iteration u - 1 have landed (3 activation slots: its
+    // activations, the first it issued, too)
+    wait_vmcnt<C::XS == 4 ? NXMIN + 1 : 1>();
+    lds_barrier();
+    const int nn = C::NIT == 1 || (u & 1) ? (ns == 2 ? 0 : ns + 1) : ns;  // of iteration u + 1
+    const int nd = C::NIT == 1 ? ns : (ns == 0 ? 2 : ns - 1);              // (u + 3) % 3 / (u / 2 + 2) % 3
+    const int s1 = ((u + 1) / C::SIT) & 1, sd = (u / C::SIT + 1) & 1;
+    const int x1 = xs == C::XS - 1 ? 0 : xs + 1;
+    iter(lds, lds, xs, x1, nn, s1, xs == 0 ? C::XS - 1 : xs - 1, nd, sd, u);
+    xs = x1;
+    ns = nn;
+  }
+  // the transfers issued past the last iteration land before the LDS is reused or released
+  wait_vmcnt<0>();
+  lds_barrier();
+
+  // sums of the K groups: group g and g ^ (KG / 2) exchange halves of their tiles, then (KG =
+  // 4) g and g ^ 1 halves of what is left; every group ends with 2 TI / KG tiles of the sum
+  // (each exchange is one fp32 addition of the same two values in either order: the same
+  // bits whichever wave adds them)
+  constexpr int LEFT = 2 * TI / KG;
+  static_assert(LEFT >= 1, "tiles per group");
+  auto put = [&](int cnt, int from) __attribute__((always_inline)) {
+#pragma unroll
+    for (int t = 0; t < cnt; ++t)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const tl_f16x_t& v = acc[from + t];
+        *(__attribute__((address_space(3))) tl_f4_t*)(lds + ((wave * cnt + t) * 4 + r) * 1024 + lane * 16) =
+            (tl_f4_t){v[4 * r], v[4 * r + 1], v[4 * r + 2], v[4 * r + 3]};
+      }
+  };
+  auto add = [&](int cnt, int from, int partner) __attribute__((always_inline)) {
+#pragma unroll
+    for (int t = 0; t < cnt; ++t)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const tl_f4_t v =
+            *(const __attribute__((address_space(3))) tl_f4_t*)(lds + ((partner * cnt + t) * 4 + r) * 1024 + lane * 16);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) acc[t][4 * r + e] = acc[from + t][4 * r + e] + v[e];
+      }
+  };
+  int f0 = 0;  // first tile this group holds
+  if (g < KG / 2) {
+    put(TI, TI);
+    lds_barrier();
+    add(TI, 0, wave ^ 4);
+  } else {
+    put(TI, 0);
+    lds_barrier();
+    add(TI, TI, wave ^ 4);
+    f0 = TI;
+  }
+  if constexpr (KG == 4) {
+    lds_barrier();
+    if (!(g & 1)) {
+      put(TI / 2, TI / 2);
+      lds_barrier();
+      add(TI / 2, 0, wave ^ WN);
+    } else {
+      put(TI / 2, 0);
+      lds_barrier();
+      add(TI / 2, TI / 2, wave ^ WN);
+      f0 += TI / 2;
+    }
+  }
+
+  // 32 x 32 result layout: register r of lane l holds D[8 (r / 4) + 4 (l / 32) + r % 4][l % 32]
+  const size_t z0 = SPLIT ? (size_t)blockIdx.y * M * N : 0;
+  auto store = [&](bool check) __attribute__((always_inline)) {
+#pragma unroll
+    for (int t = 0; t < LEFT; ++t) {
+      const int f = f0 + t;
+      const int n = n0 + 64 * wn + 32 * (f & 1) + fr, mt = m0 + 32 * (f >> 1) + 4 * fhi;
+      const size_t o = z0 + (size_t)mt * N + n;
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        const int dm = 8 * (r >> 2) + (r & 3);
+        if (check && !(mt + dm < M && n < N)) continue;
+        store_out<OUT_DT>(out, o + (size_t)dm * N, acc[t][r]);
       }
     }
   };
-
-  // Pipeline: iteration u (one barrier) multiplies slices 2u and 2u + 1 (activation slot
-  // u % 2, raw weight slot u % 3); beside the MFMAs of slice 2u it issues the activation
-  // transfers of slices 2u + 2 and 2u + 3 (16 per thread, into the slot iteration u - 1
-  // read), beside those of slice 2u + 1 the raw weight transfers of slices 2u + 4 and
-  // 2u + 5 (4 per thread, into the slot iteration u - 1 read).  At the top of iteration u
-  // this thread's activation transfers for it and raw transfers (issued an iteration
-  // earlier still) are all but the last 4 (the raw transfers of iteration u - 1); the
-  // barrier then makes every thread's transfers visible and every read of the slots about
-  // to be refilled finished.  Prologue order raw 0-1, x 0-1, raw 2-3: the same at u = 0.
-  issue_raw(0, 0);
-  issue_raw(1, 0);
-  issue_x(0, 0);
-  issue_x(1, 0);
-  issue_raw(2, 1);
-  issue_raw(3, 1);
-
-  int xs = 0, rs = 0;  // slots of iteration u's activations and raw weights
-  for (int t = 0; t < T; t += 2) {
-    const int rs2 = rs == 0 ? 2 : rs - 1;  // (u + 2) % 3 = (u - 1) % 3
-    if (AWQ && wave == 0)
-      wait_vmcnt<6>();
-    else
-      wait_vmcnt<4>();
-    lgkm_wait();
-    __builtin_amdgcn_s_barrier();
-    __builtin_amdgcn_sched_barrier(0);
-    const uint32_t xa = lds0 + 2 * xs * TL_X, rb = lds0 + TL_R0 + 2 * rs * TL_R;
-    mma(xa, rb, [&](int kk) {
-      issue_x_part(t + 2 + (kk >> 1), xs ^ 1, (NX / 2) * (kk & 1), (NX / 2) * (kk & 1) + NX / 2);
-    });
-    mma(xa + TL_X, rb + TL_R, [&](int kk) {
-      if (kk == 0) issue_raw(t + 4, rs2);
-      if (kk == 1) issue_raw(t + 5, rs2);
-    });
-    xs ^= 1;
-    rs = rs == 2 ? 0 : rs + 1;
-  }
-  // the transfers issued past the last slice (clamped re-reads) land before the
-  // workgroup's LDS is released
-  wait_vmcnt<0>();
-  lgkm_wait();
-
-  // 32 x 32 result layout: register r of lane l holds D[8 (r / 4) + 4 (l / 32) + r % 4][l % 32]
-#pragma unroll
-  for (int i = 0; i < 4; ++i)
-#pragma unroll
-    for (int j = 0; j < TJ; ++j) {
-      const int n = n0 + 32 * (TJ * wn + j) + fr;
-#pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        const int m = m0 + 128 * wm + 32 * i + 8 * (r >> 2) + 4 * fhi + (r & 3);
-        if (m < M && n < N) {
-          if constexpr (SPLIT)
-            ((float*)out)[(size_t)blockIdx.y * M * N + (size_t)m * N + n] = acc[i][j][r];
-          else
-            store_out<OUT_DT>(out, (size_t)m * N + n, acc[i][j][r]);
-        }
-      }
-    }
+  if (m0 + BM <= M && n0 + BN <= N)
+    store(false);
+  else
+    store(true);
+#endif
 }
 
-// out[i] = sum over z = 0 .. split - 1 of part[z n + i], in that order, rounded to OUT_DT
-template <int OUT_DT>
+// out[i] = sum over z = 0 .. split - 1 of part[z n + i], in that order, rounded to OUT_DT.
+// V consecutive elements per thread (V = 4 where n is a multiple of 4: 16-byte loads).
+template <int OUT_DT, int V>
 __global__ __launch_bounds__(256) void tl_reduce_kernel(const float* __restrict__ part, void* __restrict__ out,
                                                         size_t n, int split) {
-  const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
+  const size_t i = ((size_t)blockIdx.x * 256 + threadIdx.x) * V;
   if (i >= n) return;
-  float y = part[i];
-  for (int z = 1; z < split; ++z) y += part[(size_t)z * n + i];
-  store_out<OUT_DT>(out, i, y);
+  typedef float fv_t __attribute__((ext_vector_type(V)));
+  fv_t y = *(const fv_t*)(part + i);
+#pragma unroll 4
+  for (int z = 1; z < split; ++z) y += *(const fv_t*)(part + (size_t)z * n + i);
+#pragma unroll
+  for (int e = 0; e < V; ++e) store_out<OUT_DT>(out, i + e, y[e]);
 }
 
 }  // namespace nve
 
 namespace nve_host {
 
-// The tile kernel serves K % 128 == 0 (two slices per iteration), where every byte offset
-// fits its buffer resource (2^31 - 1 bytes; reads past it would return zeros): activations
-// M K, nibbles N K / 2 and scales N K / 8 bytes (AWQ factors: 4 K).
-long gemm_tile_grid128(int M, int N) {
-  return (long)((M + 127) / 128) * ((N + nve::TL_BN - 1) / nve::TL_BN);
+// The tile kernel serves K % 128 == 0, where every byte offset fits its buffer resource
+// (activations 2 M K, nibbles N K / 2, scales N K / 8, factors 4 K bytes below 2^31), with
+// 16-byte aligned scales (its transfers take 4 scales at a time).
+bool gemm_tile_fits(int M, int N, int K, const void* sc) {
+  return K % 128 == 0 && M >= 1 && N >= 1 && (long)M * K < (1L << 30) && (long)N * (K / 2) < (1L << 31) &&
+         aligned(sc, 16);
 }
 
-// K split of a 128-row tile grid that leaves CUs idle: as many splits as keep the grid
-// within one round (256 workgroups) and at least 4 iterations (8 slices) each; *ks =
-// slices per split (even), and the returned count has no empty split.
-static int tile_split(int M, int N, int K, int* ks) {
-  const long g = gemm_tile_grid128(M, N);
-  const int kit = K / (2 * nve::TL_BK);
+// fp32 partial bytes a caller's workspace is sized for: a 128 x 128 tile grid split over K
+// while it stays within one workgroup per CU and 512 of K per split.
+size_t gemm_tile_parts_bytes(int M, int N, int K) {
+  if (!gemm_tile_fits(M, N, K, nullptr)) return 0;
+  const long g = (long)((M + 127) / 128) * ((N + 127) / 128);
+  const int kit = K / 128;
   const int by_grid = g >= 256 ? 1 : (int)(256 / g), by_k = kit / 4 > 1 ? kit / 4 : 1;
   const int split = by_grid < by_k ? by_grid : by_k;
-  const int per = 2 * ((kit + split - 1) / split);
-  if (ks) *ks = per;
-  return (2 * kit + per - 1) / per;
+  const int per = (kit + split - 1) / split, used = (kit + per - 1) / per;
+  return used > 1 ? (size_t)used * M * N * sizeof(float) : 0;
 }
 
-size_t gemm_tile_parts_bytes(int M, int N, int K) {
-  if (!gemm_tile_fits(M, N, K, false)) return 0;
-  const int split = tile_split(M, N, K, nullptr);
-  return split > 1 ? (size_t)split * M * N * sizeof(float) : 0;
-}
-
-bool gemm_tile_fits(int M, int N, int K, bool /*awq*/) {
-  return K % 128 == 0 && M >= 1 && N >= 1 && (long)M * K < (1L << 30) && (long)N * (K / 2) < (1L << 31);
-}
-
-template <bool BF16, bool AWQ, int OUT_DT, int BM, bool SPLIT = false>
-static hipError_t launch_tile_bm(const void* x, int M, const uint8_t* nib, const float* sc, const float* awq,
-                                 void* out, int N, int K, hipStream_t s, int split = 1, int ks = 0) {
-  auto kern = nve::gemm_w4a16_tile_kernel<BF16, AWQ, OUT_DT, BM, SPLIT>;
-  constexpr int lds = nve::tl_lds_bytes(BM, AWQ);
+template <bool BF16, bool AWQ, int OUT_DT, int TI, int WN, bool SPLIT>
+static hipError_t launch_tile_k(const void* x, int M, const uint8_t* nib, const float* sc, const float* awq, void* out,
+                                int N, int K, int split, int ks, hipStream_t s) {
+  using C = nve::TileCfg<TI, WN, AWQ>;
+  auto kern = nve::gemm_w4a16_tile_kernel<BF16, AWQ, OUT_DT, TI, WN, SPLIT>;
   static thread_local int attr_dev = -1;
   int dev = 0;
   hipError_t e = hipGetDevice(&dev);
   if (e != hipSuccess) return e;
   if (attr_dev != dev) {
-    e = hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+    e = hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, C::BYTES);
     if (e != hipSuccess) return e;
     attr_dev = dev;
   }
-  const int nt = (N + nve::TL_BN - 1) / nve::TL_BN, mt = (M + BM - 1) / BM;
-  hipLaunchKernelGGL(kern, dim3(nt * mt, split), dim3(256), lds, s, (const uint16_t*)x, nib, sc, awq, out, M, N, K,
-                     nt, ks);
+  const int nt = (N + C::BN - 1) / C::BN, mt = (M + C::BM - 1) / C::BM;
+  hipLaunchKernelGGL(kern, dim3(nt * mt, split), dim3(64 * nve::kTlWaves), C::BYTES, s, (const uint16_t*)x, nib, sc,
+                     awq, out, M, N, K, nt, ks);
   return hipGetLastError();
 }
 
-// 128-row tiles while their grid is one round (at most one workgroup per CU), else 256
-// (8B gate, fp16 out, us: M = 256 51.4 against 71.2 with 256-row tiles; M = 512 103.3
-// against 81.4, the 128-row grid there being 448 workgroups)
-template <bool BF16, bool AWQ, int OUT_DT>
-static hipError_t launch_tile_t(const void* x, int M, const uint8_t* nib, const float* sc, const float* awq,
-                                void* out, int N, int K, hipStream_t s) {
-  if (gemm_tile_grid128(M, N) <= 256)
-    return launch_tile_bm<BF16, AWQ, OUT_DT, 128>(x, M, nib, sc, awq, out, N, K, s);
-  return launch_tile_bm<BF16, AWQ, OUT_DT, 256>(x, M, nib, sc, awq, out, N, K, s);
+template <bool BF16, bool AWQ, int OUT_DT, bool SPLIT>
+static hipError_t launch_tile_t(const TilePlan& p, const void* x, int M, const uint8_t* nib, const float* sc,
+                                const float* awq, void* out, int N, int K, hipStream_t s) {
+  switch (p.shape) {
+    case 0: return launch_tile_k<BF16, AWQ, OUT_DT, 2, 2, SPLIT>(x, M, nib, sc, awq, out, N, K, p.split, p.ks, s);
+    case 1: return launch_tile_k<BF16, AWQ, OUT_DT, 4, 2, SPLIT>(x, M, nib, sc, awq, out, N, K, p.split, p.ks, s);
+    case 2: return launch_tile_k<BF16, AWQ, OUT_DT, 3, 4, SPLIT>(x, M, nib, sc, awq, out, N, K, p.split, p.ks, s);
+    default: return launch_tile_k<BF16, AWQ, OUT_DT, 4, 4, SPLIT>(x, M, nib, sc, awq, out, N, K, p.split, p.ks, s);
+  }
 }
 
-// With parts (parts_bytes >= gemm_tile_parts_bytes) a small grid is split over K: fp32
-// partials there, added in a fixed order and rounded to out_dt by a second launch.
-template <bool BF16, bool AWQ>
-static hipError_t launch_tile_split(const void* x, int M, const uint8_t* nib, const float* sc, const float* awq,
-                                   void* out, int out_dt, int N, int K, float* parts, int split, int ks,
-                                   hipStream_t s) {
-  hipError_t e = launch_tile_bm<BF16, AWQ, NVE_DT_F32, 128, true>(x, M, nib, sc, awq, parts, N, K, s, split, ks);
-  if (e != hipSuccess) return e;
-  const size_t n = (size_t)M * N;
-  const dim3 g((unsigned)((n + 255) / 256));
-  switch (out_dt) {
-    case NVE_DT_F16: hipLaunchKernelGGL(nve::tl_reduce_kernel<NVE_DT_F16>, g, dim3(256), 0, s, parts, out, n, split); break;
-    case NVE_DT_BF16: hipLaunchKernelGGL(nve::tl_reduce_kernel<NVE_DT_BF16>, g, dim3(256), 0, s, parts, out, n, split); break;
-    default: hipLaunchKernelGGL(nve::tl_reduce_kernel<NVE_DT_F32>, g, dim3(256), 0, s, parts, out, n, split); break;
-  }
-  return hipGetLastError();
+template <int OUT_DT>
+static void launch_reduce(const float* parts, void* out, size_t n, int split, hipStream_t s) {
+  if (n % 4 == 0 && aligned(out, OUT_DT == NVE_DT_F32 ? 16 : 8))
+    hipLaunchKernelGGL((nve::tl_reduce_kernel<OUT_DT, 4>), dim3((unsigned)((n / 4 + 255) / 256)), dim3(256), 0, s,
+                       parts, out, n, split);
+  else
+    hipLaunchKernelGGL((nve::tl_reduce_kernel<OUT_DT, 1>), dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, parts,
+                       out, n, split);
 }
 
 template <bool BF16, bool AWQ>
-static hipError_t launch_tile_x(const void* x, int M, const uint8_t* nib, const float* sc, const float* awq,
-                                void* out, int out_dt, int N, int K, float* parts, size_t parts_bytes,
-                                hipStream_t s) {
-  if (parts) {
-    int ks = 0;
-    const int split = tile_split(M, N, K, &ks);
-    if (split > 1 && parts_bytes >= (size_t)split * M * N * sizeof(float))
-      return launch_tile_split<BF16, AWQ>(x, M, nib, sc, awq, out, out_dt, N, K, parts, split, ks, s);
+static hipError_t launch_tile_x(const TilePlan& p, const void* x, int M, const uint8_t* nib, const float* sc,
+                                const float* awq, void* out, int out_dt, int N, int K, float* parts, hipStream_t s) {
+  if (p.split > 1) {
+    const hipError_t e = launch_tile_t<BF16, AWQ, NVE_DT_F32, true>(p, x, M, nib, sc, awq, parts, N, K, s);
+    if (e != hipSuccess) return e;
+    const size_t n = (size_t)M * N;
+    switch (out_dt) {
+      case NVE_DT_F16: launch_reduce<NVE_DT_F16>(parts, out, n, p.split, s); break;
+      case NVE_DT_BF16: launch_reduce<NVE_DT_BF16>(parts, out, n, p.split, s); break;
+      default: launch_reduce<NVE_DT_F32>(parts, out, n, p.split, s); break;
+    }
+    return hipGetLastError();
   }
   switch (out_dt) {
-    case NVE_DT_F16: return launch_tile_t<BF16, AWQ, NVE_DT_F16>(x, M, nib, sc, awq, out, N, K, s);
-    case NVE_DT_BF16: return launch_tile_t<BF16, AWQ, NVE_DT_BF16>(x, M, nib, sc, awq, out, N, K, s);
-    default: return launch_tile_t<BF16, AWQ, NVE_DT_F32>(x, M, nib, sc, awq, out, N, K, s);
+    case NVE_DT_F16: return launch_tile_t<BF16, AWQ, NVE_DT_F16, false>(p, x, M, nib, sc, awq, out, N, K, s);
+    case NVE_DT_BF16: return launch_tile_t<BF16, AWQ, NVE_DT_BF16, false>(p, x, M, nib, sc, awq, out, N, K, s);
+    default: return launch_tile_t<BF16, AWQ, NVE_DT_F32, false>(p, x, M, nib, sc, awq, out, N, K, s);
   }
 }
 
-hipError_t launch_gemm_w4a16_tile(const void* x, int x_dt, int M, const uint8_t* nib, const float* sc,
-                                  const float* awq, void* out, int out_dt, int N, int K, float* parts,
-                                  size_t parts_bytes, hipStream_t s) {
-  if (K % (2 * nve::TL_BK) != 0) return hipErrorInvalidValue;
+hipError_t launch_gemm_w4a16_tile(const TilePlan& p, const void* x, int x_dt, int M, const uint8_t* nib,
+                                  const float* sc, const float* awq, void* out, int out_dt, int N, int K,
+                                  float* parts, hipStream_t s) {
   const bool bf = x_dt == NVE_DT_BF16;
   if (awq)
-    return bf ? launch_tile_x<true, true>(x, M, nib, sc, awq, out, out_dt, N, K, parts, parts_bytes, s)
-              : launch_tile_x<false, true>(x, M, nib, sc, awq, out, out_dt, N, K, parts, parts_bytes, s);
-  return bf ? launch_tile_x<true, false>(x, M, nib, sc, awq, out, out_dt, N, K, parts, parts_bytes, s)
-            : launch_tile_x<false, false>(x, M, nib, sc, awq, out, out_dt, N, K, parts, parts_bytes, s);
+    return bf ? launch_tile_x<true, true>(p, x, M, nib, sc, awq, out, out_dt, N, K, parts, s)
+              : launch_tile_x<false, true>(p, x, M, nib, sc, awq, out, out_dt, N, K, parts, s);
+  return bf ? launch_tile_x<true, false>(p, x, M, nib, sc, awq, out, out_dt, N, K, parts, s)
+            : launch_tile_x<false, false>(p, x, M, nib, sc, awq, out, out_dt, N, K, parts, s);
 }
 
 }  // namespace nve_host

@@ -157,6 +157,38 @@ def test_gemm_w4a16_tile_weights_match_dequant_exactly(orc, torch_dev, hk, m, n,
                               np.ascontiguousarray(wref[:, ks].T).view(np.uint32))
 
 
+@pytest.mark.parametrize("m,n,k,ws", [(40, 14336, 256, True), (65, 2000, 640, True), (64, 4100, 8192, True),
+                                      (250, 14336, 384, False), (300, 14340, 128, False), (512, 14336, 640, False),
+                                      (257, 2100, 8320, True), (300, 4096, 9088, True), (130, 120, 2176, True)])
+@pytest.mark.parametrize("xdt,with_awq", [("f16", False), ("bf16", True)])
+def test_gemm_w4a16_tile_shapes_exact(orc, torch_dev, hk, m, n, k, ws, xdt, with_awq):
+    """The tile kernel's shapes, unsplit and split over K (64 x 128 at 40 x 14336 and 65 x 2000, 128 x 128
+    at 250 x 14336, 96 x 256 at 300 x 14340, 128 x 256 at 512 x 14336; split by the workspace at the others),
+    with ragged rows and columns, K of one and of three iterations, K that is no multiple of 512
+    (a partial last scale slot) and splits whose last part is shorter.  One-hot activation rows: every
+    output is one weight as the reference dequant rounds it, compared bit for bit, also
+    after other data has been through the workspace."""
+    torch = torch_dev
+    print(f"tile shapes m={m} n={n} k={k} ws={ws} x={xdt} awq={with_awq}", flush=True)
+    data = orc.q4_from_f32(weights(n, k, seed=m + k, std=0.3))
+    nib, sc = orc.extract_for_gpu(data, n, k)
+    awq = np.random.default_rng(n + m).uniform(0.5, 2.0, k).astype(np.float32) if with_awq else None
+    wref = _round(orc.q4_to_f32(data, n, k, awq), xdt)
+    ks = np.random.default_rng(m + n).integers(0, k, m)
+    ks[:2] = 0, k - 1
+    tdt = torch.float16 if xdt == "f16" else torch.bfloat16
+    x = torch.zeros((m, k), dtype=tdt, device="cuda")
+    x[torch.arange(m, device="cuda"), torch.from_numpy(ks).cuda()] = 1
+    tn, ts = torch.from_numpy(nib).cuda(), torch.from_numpy(sc).cuda()
+    ta = None if awq is None else torch.from_numpy(awq).cuda()
+    w = torch.full((hk.gemm_w4a16_workspace_bytes(m, n, k),), 0xFF, dtype=torch.uint8, device="cuda") if ws else None
+    want = np.ascontiguousarray(wref[:, ks].T)
+    for odt in (torch.float32, tdt):
+        y = hk.gemm_w4a16_ws(x, tn, ts, n, k, w, ta, out_dtype=odt)
+        torch.cuda.synchronize()
+        assert np.array_equal(y.float().cpu().numpy(), want)
+
+
 def test_gemm_w4a16_tile_wide_n_exact(orc, torch_dev, hk):
     """The tile kernel at an lm_head-wide N (128256 rows of weights, 1002 column tiles):
     at M = 300 its 256-row grid is 2 x 1002 workgroups, about eight rounds on 256 CUs,
