@@ -228,7 +228,7 @@ int nve_hip_dequant_w4(const uint8_t *nibbles, const float *scales, const float 
  * rounds it (to x's dtype: F16 as the reference, or BF16) and the products accumulate
  * in fp32 on MFMA (M <= 32, and up to 320 (128 with awq) where estimated faster:
  * weight-streaming kernels, where K % 128 == 0 and N <= 16384 an LDS ring in launches of up
- * to 64 rows (32 with awq), else M <= 16 only; with K % 128 == 0 tiles of 64-128 x 128-256 with
+ * to 64 rows (48 with awq), else M <= 16 only; with K % 128 == 0 tiles of 64-128 x 128-256 with
  * the weights dequantized in registers; otherwise 128 x 128 tiles dequantized in LDS).  x [M, K]
  * row-major F16/BF16 (16-byte aligned); awq [K] or NULL; out [M, N] row-major F16,
  * BF16 or F32.  K % 64 == 0.  Bit-reproducible: the same inputs give the same bits on

@@ -421,8 +421,8 @@ __global__ __launch_bounds__(64 * KS) void gemm_w4a16_ring_kernel(const uint16_t
                                                                int rows_per_wg) {
   static_assert(S >= 1 && S <= 2, "ring depth");
   using L = W16Ring<T, EU, AWQ>;
-  // EU activation transfers of 4 rows: up to 16 rows form one A operand group, 32 / 64
-  // rows (EU = 8 / 16) two / four groups that share every dequantized weight fragment
+  // EU activation transfers of 4 rows: up to 16 rows form one A operand group, 32 / 48 /
+  // 64 rows (EU = 8 / 12 / 16) two / three / four groups that share every dequantized weight fragment
   constexpr int MG = EU > 4 ? EU / 4 : 1, EG = EU > 4 ? 4 : EU;
   constexpr int kRing = KS * S * L::SLOT;
   constexpr int kRed = KS * T * 16 * (4 * EU + 1) * 4;
@@ -707,7 +707,7 @@ static hipError_t launch_small_o(const void* x, int M, const uint8_t* nib, const
   return hipGetLastError();
 }
 
-// M <= 64 (32 with AWQ), K % 128 == 0, N <= 16384: the LDS-ring kernel, ceil(N / 256)
+// M <= 64 (48 with AWQ), K % 128 == 0, N <= 16384: the LDS-ring kernel, ceil(N / 256)
 // rows per workgroup (16 below 4096 rows), one activation transfer per 4 rows of M.
 template <bool BF16, bool AWQ, int OUT_DT, int T>
 static hipError_t launch_ring_t(const void* x, int M, const uint8_t* nib, const float* sc, const float* awq, void* out,
@@ -716,17 +716,21 @@ static hipError_t launch_ring_t(const void* x, int M, const uint8_t* nib, const 
   // 16 waves, one quad in flight each (8B gate, fp16 x, M = 1 / 4 / 16: 12.1 / 11.9-12.1 /
   // 12.5-12.8 us; 8 waves with two quads in flight 12.6 / 12.5-12.6 / 13.3-13.4, 8 waves
   // with one 13.4-13.7 / 13.1 / 13.9-14.0)
-  // M = 17-32 / 33-64: two / four 16-row operand groups per dequantized weight fragment;
-  // their 8 / 16 KiB of activation rows per slot leave LDS for 8 / 6 waves (four groups
-  // without AWQ only: with it the kernel needs more than 256 VGPRs)
+  // M = 17-32 / 33-48 / 49-64: two / three / four 16-row operand groups per dequantized weight
+  // fragment; their 8 / 12 / 16 KiB of activation rows per slot leave LDS for 8 waves (7 with
+  // four groups and four weight tiles).  More waves do not help where they fit, fewer cost a
+  // round of quads (fp16, us: 8B q / gate at M = 48 with 48-row slots, 6 / 8 / 10-11 waves 8.9 / 7.9 / 8.4-8.9
+  // and 19.8 / 16.2, with 64-row slots and 6 waves 9.8 and 20.5; at M = 64 6 / 8 (gate: 7) waves 10.2 / 9.3
+  // and 21.6 / 19.6).  Four groups without AWQ only: with it the kernel needs more than 256 VGPRs.
 #define NVE_R16(EU, KS) \
   hipLaunchKernelGGL((nve::gemm_w4a16_ring_kernel<BF16, AWQ, OUT_DT, T, EU, KS, 1>), grid, dim3(64 * KS), 0, s, \
                      (const uint16_t*)x, nib, sc, awq, out, M, N, K, rpw)
   if (M <= 4) NVE_R16(1, 16);
   else if (M <= 8) NVE_R16(2, 16);
   else if (M <= 16) NVE_R16(4, 16);
-  else if (AWQ || M <= 32) NVE_R16(8, 8);
-  else if constexpr (!AWQ) NVE_R16(16, 6);
+  else if (M <= 32) NVE_R16(8, 8);
+  else if (AWQ || M <= 48) NVE_R16(12, 8);
+  else if constexpr (!AWQ) NVE_R16(16, (T == 4 ? 7 : 8));
 #undef NVE_R16
   return hipGetLastError();
 }
@@ -743,24 +747,25 @@ static hipError_t launch_ring_o(const void* x, int M, const uint8_t* nib, const 
 }
 
 // rows one ring launch takes (without / with AWQ) and the M up to which launches of that
-// many rows beat the tiled kernel
-static int ring_rows(bool awq) { return awq ? 32 : 64; }
-// 8B gate, 64-row launches: 62.5 / 83.0 / 103.7 / 124.5 us at M = 192 / 256 / 320 / 384
-// against 76.7 / 88.1 / 109.8 / 116.4 for the tiled kernel; 32-row launches (AWQ) stop
-// winning above 128 rows
+// many rows beat the 128 x 128-tile kernel of this file (8B gate, 64-row launches: 62.5 / 83.0 / 103.7 /
+// 124.5 us at M = 192 / 256 / 320 / 384 against 76.7 / 88.1 / 109.8 / 116.4)
+static int ring_rows(bool awq) { return awq ? 48 : 64; }
 static int ring_chunked_max(bool awq) { return awq ? 128 : 320; }
 // Estimated us of the ring launches of M rows: 2.6 each and, per round of the waves' quads,
-// 0.7 and 0.6 per 16-row weight tile (33 to 64 rows, 6 waves; measured at M = 40: 8B q / gate /
-// down 10.4 / 21 / 28, 2048 x 2048 6.4, 8192 x 2048 8.9, 3072 x 8192 16.2), up to 32 rows (8 waves)
-// 0.6 and 0.58, with AWQ 0.4 and 0.8 (32 rows: q 7.3, gate 17, down 19.3; up to 16 rows 16 waves).
+// a and b per 16-row weight tile, for up to 32, 48 and 64 rows (fp16: q / gate / down 7.2 / 14.1 / 18.5,
+// 7.8 / 15.9 / 19.7 and 9.3 / 19.6 / 25.9 us; with AWQ up to 32 and 48 rows 7.0 / 16.7 / 18.5 and
+// 8.3 / 17.7 / 21.8).
 static double ring_us(int M, int N, int K, bool awq) {
   const int rows = ring_rows(awq), T = N <= 4096 ? 1 : ((N + 255) / 256 + 15) / 16, nq = K / 128;
-  const int full = M / rows, rest = M % rows;
+  const int launches = (M + rows - 1) / rows, step = awq ? (M + launches - 1) / launches : rows;
+  const int full = M / step, rest = M % step;
   auto one = [&](int m) {
-    if (awq) return 2.6 + (m > 16 ? (nq + 7) / 8 : (nq + 15) / 16) * (0.4 + 0.8 * T);
-    return m > 32 ? 2.6 + (nq + 5) / 6 * (0.7 + 0.6 * T) : 2.6 + (nq + 7) / 8 * (0.6 + 0.58 * T);
+    const int waves = m <= 16 ? 16 : m > 48 && T == 4 ? 7 : 8;
+    const double a = awq ? (m <= 32 ? 0.4 : 0.62) : m <= 32 ? 0.58 : m <= 48 ? 0.65 : 1.0;
+    const double b = awq ? 0.79 : m <= 32 ? 0.57 : 0.65;
+    return 2.6 + (nq + waves - 1) / waves * (a + b * T);
   };
-  return full * one(rows) + (rest ? one(rest) : 0.0);
+  return full * one(step) + (rest ? one(rest) : 0.0);
 }
 static bool ring_fits(int M, int N, int K, bool awq) {
   return M <= ring_rows(awq) && K % 128 == 0 && N <= 16384;
@@ -788,9 +793,9 @@ hipError_t launch_gemm_w4a16_parts(const void* x, int x_dt, int M, const uint8_t
                                    size_t parts_bytes, hipStream_t s) {
   const bool bf = x_dt == NVE_DT_BF16;
   // K % 128 == 0, more than 32 rows: the tile kernel (gemm_w4a16_tile.hip) unless the ring's
-  // launches are estimated faster (narrow outputs up to 64 rows; without a workspace to split K
-  // also some more): workspace path, fp16, us, ring / tile: 8B gate M = 48 21.2 / 19.9, down 27.6 /
-  // 20.5, k_proj 9.3 / 10.1, q_proj 10.6 / 13.5; two ring launches at M = 100: gate 40.6 / 26.2.
+  // launches are estimated faster (up to 48 rows, to 64 but for long K; without a workspace to split K
+  // also some more): workspace path, fp16, us, ring / tile: 8B gate M = 48 16.2 / 19.9, down 19.7 /
+  // 20.5, k_proj 7.4 / 10.1, q_proj 7.9 / 13.5; two ring launches at M = 100: gate 33 / 25.7.
   // The split is planned within the workspace's canonical size, so that it does not vary with
   // what a caller passes beyond it.
   const int rr = ring_rows(awq != nullptr);
@@ -803,14 +808,15 @@ hipError_t launch_gemm_w4a16_parts(const void* x, int x_dt, int M, const uint8_t
     if (!ring_chunks || p.us < 0.93 * ring_us(M, N, K, awq != nullptr))
       return launch_gemm_w4a16_tile(p, x, x_dt, M, nib, sc, awq, out, out_dt, N, K, parts, s);
   }
-  // up to M = 320 (AWQ: 128) where the ring fits: ring launches of up to 64 (AWQ: 32)
-  // activation rows each (8B gate, 32-row launches: 27 us at M = 48 and about 58 us at 128, against
-  // 45 / 71 us for the tiled kernel); a row's result does not depend on the rows
-  // launched with it
+  // up to M = 320 (AWQ: 128) where the ring fits: ring launches of up to 64 (AWQ: 48)
+  // activation rows each; a row's result does not depend on the rows launched with it
   if (M > rr && ring_chunks) {
     const size_t osz = out_dt == NVE_DT_F32 ? 4 : 2;
-    for (int m0 = 0; m0 < M; m0 += rr) {
-      const int mc = M - m0 < rr ? M - m0 : rr;
+    // with AWQ equal launches (a short last one costs nearly as much: M = 64 as 48 + 16 39.5 us at the
+    // 8B gate, as 32 + 32 32.9), without it full ones and the rest
+    const int launches = (M + rr - 1) / rr, step = awq ? (M + launches - 1) / launches : rr;
+    for (int m0 = 0; m0 < M; m0 += step) {
+      const int mc = M - m0 < step ? M - m0 : step;
       const void* xc = (const char*)x + (size_t)m0 * K * 2;
       void* oc = (char*)out + (size_t)m0 * N * osz;
       hipError_t e;

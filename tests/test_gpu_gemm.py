@@ -189,6 +189,34 @@ def test_gemm_w4a16_tile_shapes_exact(orc, torch_dev, hk, m, n, k, ws, xdt, with
         assert np.array_equal(y.float().cpu().numpy(), want)
 
 
+@pytest.mark.parametrize("m", [33, 48, 49, 64, 96, 100])
+@pytest.mark.parametrize("n,k", [(70, 1024), (4100, 1152), (8200, 896), (12300, 1152)])
+@pytest.mark.parametrize("xdt,with_awq", [("f16", False), ("bf16", True)])
+def test_gemm_w4a16_ring_row_groups_exact(orc, torch_dev, hk, m, n, k, xdt, with_awq):
+    """The LDS-ring kernel's 48- and 64-row slots with one to four weight tiles per workgroup, at the edges of
+    their row ranges and in several launches (with AWQ equal ones: 49 rows as 25 + 24), with
+    7 to 9 quads of K for 7 or 8 waves.  The scales start 4 bytes off a 16-byte boundary,
+    which keeps the calls off the tile kernel.  One-hot activation rows: every output is
+    one weight as the reference dequant rounds it, compared bit for bit."""
+    torch = torch_dev
+    print(f"ring rows m={m} n={n} k={k} x={xdt} awq={with_awq}", flush=True)
+    data = orc.q4_from_f32(weights(n, k, seed=n + k, std=0.3))
+    nib, sc = orc.extract_for_gpu(data, n, k)
+    awq = np.random.default_rng(n + m).uniform(0.5, 2.0, k).astype(np.float32) if with_awq else None
+    wref = _round(orc.q4_to_f32(data, n, k, awq), xdt)
+    ks = np.random.default_rng(m + n).integers(0, k, m)
+    ks[:2] = 0, k - 1
+    tdt = torch.float16 if xdt == "f16" else torch.bfloat16
+    x = torch.zeros((m, k), dtype=tdt, device="cuda")
+    x[torch.arange(m, device="cuda"), torch.from_numpy(ks).cuda()] = 1
+    ts = torch.empty(sc.size + 1, dtype=torch.float32, device="cuda")[1:].view(n, k // 32)
+    ts.copy_(torch.from_numpy(sc).view(n, k // 32))
+    ta = None if awq is None else torch.from_numpy(awq).cuda()
+    y = hk.gemm_w4a16(x, torch.from_numpy(nib).cuda(), ts, n, k, ta, out_dtype=torch.float32)
+    torch.cuda.synchronize()
+    assert np.array_equal(y.cpu().numpy().view(np.uint32), np.ascontiguousarray(wref[:, ks].T).view(np.uint32))
+
+
 def test_gemm_w4a16_tile_wide_n_exact(orc, torch_dev, hk):
     """The tile kernel at an lm_head-wide N (128256 rows of weights, 1002 column tiles):
     at M = 300 its 256-row grid is 2 x 1002 workgroups, about eight rounds on 256 CUs,
