@@ -725,9 +725,14 @@ static hipError_t launch_ring_t(const void* x, int M, const uint8_t* nib, const 
 #define NVE_R16(EU, KS) \
   hipLaunchKernelGGL((nve::gemm_w4a16_ring_kernel<BF16, AWQ, OUT_DT, T, EU, KS, 1>), grid, dim3(64 * KS), 0, s, \
                      (const uint16_t*)x, nib, sc, awq, out, M, N, K, rpw)
-  if (M <= 4) NVE_R16(1, 16);
-  else if (M <= 8) NVE_R16(2, 16);
-  else if (M <= 16) NVE_R16(4, 16);
+  // With AWQ four weight tiles (three with 16 rows) need more than the 128 VGPRs of 16 waves and
+  // spilled there (14-21 registers): 12 waves have 168 (fp16, us, M = 1 / 6 / 16: 8B gate 19.5 / 19.2 / 21.4
+  // -> 13.5 / 13.7 / 14.2, 8 waves 15.1 / 15.1 / 15.4; 12000 x 4096, three tiles, 11.3 / 11.2 / 14.0 with 16 waves
+  // and 11.7 / 11.6 / 11.7 with 12).
+  constexpr int KF = AWQ && T == 4 ? 12 : 16, K16 = AWQ && T >= 3 ? 12 : 16;
+  if (M <= 4) NVE_R16(1, KF);
+  else if (M <= 8) NVE_R16(2, KF);
+  else if (M <= 16) NVE_R16(4, K16);
   else if (M <= 32) NVE_R16(8, 8);
   else if (AWQ || M <= 48) NVE_R16(12, 8);
   else if constexpr (!AWQ) NVE_R16(16, (T == 4 ? 7 : 8));
@@ -760,7 +765,7 @@ static double ring_us(int M, int N, int K, bool awq) {
   const int launches = (M + rows - 1) / rows, step = awq ? (M + launches - 1) / launches : rows;
   const int full = M / step, rest = M % step;
   auto one = [&](int m) {
-    const int waves = m <= 16 ? 16 : m > 48 && T == 4 ? 7 : 8;
+    const int waves = m <= 16 ? (awq && T >= 3 ? 12 : 16) : m > 48 && T == 4 ? 7 : 8;
     const double a = awq ? (m <= 32 ? 0.4 : 0.62) : m <= 32 ? 0.58 : m <= 48 ? 0.65 : 1.0;
     const double b = awq ? 0.79 : m <= 32 ? 0.57 : 0.65;
     return 2.6 + (nq + waves - 1) / waves * (a + b * T);

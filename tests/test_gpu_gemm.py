@@ -217,6 +217,30 @@ def test_gemm_w4a16_ring_row_groups_exact(orc, torch_dev, hk, m, n, k, xdt, with
     assert np.array_equal(y.cpu().numpy().view(np.uint32), np.ascontiguousarray(wref[:, ks].T).view(np.uint32))
 
 
+@pytest.mark.parametrize("m", [1, 4, 5, 8, 16])
+@pytest.mark.parametrize("n,k", [(8200, 1536), (12300, 1408), (12300, 1664)])
+@pytest.mark.parametrize("xdt", ["f16", "bf16"])
+def test_gemm_w4a16_ring_awq_few_rows_exact(orc, torch_dev, hk, m, n, k, xdt):
+    """Up to 16 rows with AWQ and three or four weight tiles per workgroup: 12 waves (three tiles
+    up to 8 rows: 16) share 11, 12 or 13 quads of K, one short of a round, a round and one
+    more.  One-hot activation rows: every output is one weight as the reference dequant
+    rounds it, compared bit for bit."""
+    torch = torch_dev
+    print(f"ring awq m={m} n={n} k={k} x={xdt}", flush=True)
+    data = orc.q4_from_f32(weights(n, k, seed=n + k, std=0.3))
+    nib, sc = orc.extract_for_gpu(data, n, k)
+    awq = np.random.default_rng(n + m).uniform(0.5, 2.0, k).astype(np.float32)
+    wref = _round(orc.q4_to_f32(data, n, k, awq), xdt)
+    ks = np.append(np.random.default_rng(m + n).integers(0, k, m - 1), k - 1)
+    tdt = torch.float16 if xdt == "f16" else torch.bfloat16
+    x = torch.zeros((m, k), dtype=tdt, device="cuda")
+    x[torch.arange(m, device="cuda"), torch.from_numpy(ks).cuda()] = 1
+    y = hk.gemm_w4a16(x, torch.from_numpy(nib).cuda(), torch.from_numpy(sc).cuda(), n, k,
+                      torch.from_numpy(awq).cuda(), out_dtype=torch.float32)
+    torch.cuda.synchronize()
+    assert np.array_equal(y.cpu().numpy().view(np.uint32), np.ascontiguousarray(wref[:, ks].T).view(np.uint32))
+
+
 def test_gemm_w4a16_tile_wide_n_exact(orc, torch_dev, hk):
     """The tile kernel at an lm_head-wide N (128256 rows of weights, 1002 column tiles):
     at M = 300 its 256-row grid is 2 x 1002 workgroups, about eight rounds on 256 CUs,
