@@ -2,10 +2,11 @@
 //
 // GpuWeight::matmul_x (src/gpu_layer.rs:219-237) expands the int4 weights to a dense
 // 16-bit matrix with nve_dequant_w4a16 and multiplies with the vendor GEMM.  The fused
-// kernels (gemm_w4a16.hip, gemm_w4a16_tile.hip) win up to M = 512; they re-dequantize
-// each weight slice once per activation row block, so above M = 512 the reference's
+// kernels (gemm_w4a16.hip, gemm_w4a16_tile.hip) win up to M = 512 and, where the weight
+// matrix is narrow for the chip, well above; they re-dequantize
+// each weight slice once per activation row block, so for many rows the reference's
 // two-step method is the faster one on this part.  nve_hip_gemm_w4a16_ws
-// takes that path when the caller provides the workspace: the weights are dequantized
+// takes that path there when the caller provides the workspace: the weights are dequantized
 // into it (dequant_w4_kernel, bit-identical to the reference dequant) and hipBLASLt
 // computes Y = X W^T with fp32 accumulation.  Column-major view: D (N x M, ld N) =
 // op(A) op(B) with A = the dequantized W seen as K x N (ld K, transposed) and B = X
@@ -17,6 +18,7 @@
 #include <tuple>
 
 #include "common.h"
+#include "gemm_tile_plan.h"
 #include "w4_launch.h"
 
 namespace nve_host {
@@ -32,13 +34,26 @@ size_t gemm_split_parts_bytes(int M, int N, int K);
 
 namespace {
 
-// from here on dequant + GEMM is faster (fp16 out, us: 8B gate M = 640 96.8 against 145.9
-// for the tile kernel, 8B down 116.2 against 135.5; at M = 384-512 the two are within 10%,
-// the tile kernel ahead at down); with AWQ factors from 385 rows, where the tile kernel's
-// extra multiply and factor reads put it behind at the gate (fp32 out, M = 512: 88.0 against
-// 80.8; down 103.1 against 104.5)
+// dequant + GEMM is considered from these rows on (with AWQ factors from 385)
 constexpr int kGemmBlasMinM = 513;
 constexpr int kGemmBlasMinMAwq = 385;
+
+// Whether the tile kernel serves a product that dequant + GEMM could: its planned time against
+// 11.6 us + 0.635 us per 10^6 weights (the dequant and reading its output) + 0.573 us per GFLOP + 1.5 us
+// per 1000 of K, fitted to 364 timed products (12 layer shapes, N 512-14336, K 2048-14336, M =
+// 400-2048, with and without AWQ, fp16 and bf16; rms error 6%), with 8% for the estimates' error.
+// us, dequant + GEMM / tile kernel, fp16: 8B down M = 520 / 1024 112.8 / 91.6 and 148.1 / 122.7 (M = 1280
+// 163.1 / 182.6, stays), q 640 / 1024 40.5 / 32.8 and 47.1 / 39.8, 2048 x 2048 M = 1024 23.8 / 16.5; AWQ, M = 512,
+// down 109.3 / 79.1, q 38.4 / 33.4; gate M = 640 96.6 / 104.7 (stays).  Only over the sizes timed: from 2 Mi
+// weights (below, 9-20 us a product, the two differ by 1-3 us either way), to 64 Mi and 2048 rows.
+bool fused_faster(int M, int N, int K, bool awq, const float* sc, size_t ws_bytes) {
+  const double nk = (double)N * K;
+  if (M > 2048 || nk < 2 * 1024 * 1024 || nk > 64.0 * 1024 * 1024 || !gemm_tile_fits(M, N, K, sc)) return false;
+  const size_t room = gemm_split_parts_bytes(M, N, K);
+  const size_t most = ws_bytes >= room ? room / ((size_t)M * N * sizeof(float)) : 1;
+  const double blas = 11.6 + 0.635e-6 * nk + 0.573e-9 * 2 * M * nk + 1.5e-3 * K;
+  return plan_gemm_tile(M, N, K, awq, most > 1 ? (int)most : 1).us < 0.92 * blas;
+}
 constexpr size_t kBlasWorkspace = 32u << 20;
 constexpr int kBlasCandidates = 32;  // heuristic candidates timed on the first call per shape
 constexpr int kBlasTimedRuns = 5;    // timed runs per candidate (after one untimed run)
@@ -146,7 +161,7 @@ AlgoChoice select_algo(hipblasLtHandle_t h, const Descs& ds, const void* x, void
 
 // Below kGemmBlasMinMAwq: the fp32 partials of the fused kernels' K split (0 when that
 // shape does not split); from it on also room for the dequantized weights + the hipBLASLt
-// workspace (used from kGemmBlasMinM, or kGemmBlasMinMAwq with AWQ factors).
+// workspace (used from kGemmBlasMinM, or kGemmBlasMinMAwq with AWQ factors, unless fused_faster).
 size_t gemm_w4a16_ws_bytes(int M, int N, int K) {
   if (M < kGemmBlasMinMAwq) return round256(gemm_split_parts_bytes(M, N, K));
   const size_t blas = round256((size_t)N * K * 2) + kBlasWorkspace;
@@ -155,8 +170,8 @@ size_t gemm_w4a16_ws_bytes(int M, int N, int K) {
 }
 
 // Dequant + hipBLASLt when M >= kGemmBlasMinM (kGemmBlasMinMAwq with AWQ factors), the
-// workspace is large enough and the output is F32 or x's dtype; otherwise the fused
-// kernel.  The first call per device and
+// workspace is large enough, the output is F32 or x's dtype and the tile kernel is not
+// estimated faster; otherwise the fused kernel.  The first call per device and
 // shape creates the hipBLASLt handle and picks the fastest of up to kBlasCandidates
 // heuristic algorithms by timing them on the caller's stream; under graph capture a
 // device or shape without that state takes the fused kernel instead.
@@ -170,7 +185,9 @@ hipError_t launch_gemm_w4a16_ws(const void* x, int x_dt, int M, const uint8_t* n
   };
   const int blas_min = awq ? kGemmBlasMinMAwq : kGemmBlasMinM;
   const size_t need = M >= blas_min ? round256((size_t)N * K * 2) + kBlasWorkspace : 0;
-  if (need == 0 || ws == nullptr || ws_bytes < need || (out_dt != NVE_DT_F32 && out_dt != x_dt)) return fused();
+  if (need == 0 || ws == nullptr || ws_bytes < need || (out_dt != NVE_DT_F32 && out_dt != x_dt) ||
+      fused_faster(M, N, K, awq != nullptr, sc, ws_bytes))
+    return fused();
   int dev = 0;
   hipError_t e = hipGetDevice(&dev);
   if (e != hipSuccess) return e;

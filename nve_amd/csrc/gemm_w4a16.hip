@@ -15,10 +15,11 @@
 // flop of 16 x 16 tiles); K advances 64 per slice (two Q4 blocks).  The global
 // loads (X rows, nibbles, scales) run two slices ahead of the MFMAs and the LDS is
 // double-buffered, so the dequantization of slice t+1 overlaps the MFMAs of slice t and
-// HBM latency overlaps the math; launches with few output tiles also split K over
-// workgroups (fp32 atomic accumulation).  LDS rows are padded (72 elements) so the
-// ds_read_b128 of a fragment spreads over the banks.  M <= 16 runs a separate
-// weight-streaming kernel (gemm_w4a16_small_kernel below).
+// HBM latency overlaps the math; with a workspace, launches with few output tiles also
+// split K over workgroups (fp32 partials, added in a fixed order).  LDS rows are padded (72
+// elements) so the ds_read_b128 of a fragment spreads over the banks.  Few rows run separate
+// weight-streaming kernels (gemm_w4a16_small_kernel and gemm_w4a16_ring_kernel below); where K % 128 == 0
+// the kernel of gemm_w4a16_tile.hip takes the tiled product.
 
 #include "common.h"
 #include "lds_ring.h"
@@ -401,8 +402,8 @@ __global__ __launch_bounds__(64 * KS) void gemm_w4a16_small_kernel(const uint16_
 // the two 8-byte k-runs {4g..4g+3} and {16+4g..16+4g+3} of the activation row.  The
 // nibbles are extracted low / high per byte, which yields that same k order, so the B
 // operand (the reference dequant f16/bf16(fma(n, s, -8 s)), as above) needs no permute.
-// KS waves with S quads in flight each (the launcher: 16 waves, one quad; 8 waves where
-// 32 activation rows form two operand groups); workgroups take ceil(N / 256) rows each
+// KS waves with S quads in flight each (the launcher: one quad, 16 waves, or as many as the
+// registers and the LDS hold); workgroups take ceil(N / 256) rows each
 // (one per CU), the last tile partly masked (masked lanes issue no transfers; lane 0
 // always does, so every wave instruction counts once and the vmcnt waits are exact).
 template <int T, int EU, bool AWQ>

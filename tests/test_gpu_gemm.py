@@ -320,6 +320,35 @@ def _ws_blas_check(orc, torch_dev, hk, m, n, k, xdt, with_awq):
     assert rel_err_floor(y16, ref) <= 2e-3 + (2.0 ** -8 if xdt == "bf16" else 2.0 ** -11)
 
 
+@pytest.mark.parametrize("m,n,k,awq", [(400, 1024, 2048, True), (513, 1024, 2048, False), (640, 1024, 4096, True),
+                                       (1024, 2100, 1024, False), (2048, 520, 4096, False), (520, 4100, 512, True)])
+@pytest.mark.parametrize("xdt", ["f16", "bf16"])
+def test_gemm_w4a16_ws_many_rows_fused_exact(orc, torch_dev, hk, m, n, k, awq, xdt):
+    """From 2 Mi weights nve_hip_gemm_w4a16_ws with its whole workspace takes the tile kernel (its K split
+    in the workspace) also above the rows from which it otherwise dequantizes and calls
+    the library GEMM, where it is estimated faster.  One-hot activation rows: every output is one
+    weight as the reference dequant rounds it, on either route, compared bit for bit, fp32 and
+    x's type out, also after other data has been through the workspace."""
+    torch = torch_dev
+    print(f"ws many rows m={m} n={n} k={k} awq={awq} x={xdt}", flush=True)
+    data = orc.q4_from_f32(weights(n, k, seed=m + k, std=0.3))
+    nib, sc = orc.extract_for_gpu(data, n, k)
+    a = np.random.default_rng(n + m).uniform(0.5, 2.0, k).astype(np.float32) if awq else None
+    wref = _round(orc.q4_to_f32(data, n, k, a), xdt)
+    ks = np.random.default_rng(m + n).integers(0, k, m)
+    ks[:2] = 0, k - 1
+    tdt = torch.float16 if xdt == "f16" else torch.bfloat16
+    x = torch.zeros((m, k), dtype=tdt, device="cuda")
+    x[torch.arange(m, device="cuda"), torch.from_numpy(ks).cuda()] = 1
+    ws = torch.full((hk.gemm_w4a16_workspace_bytes(m, n, k),), 0xFF, dtype=torch.uint8, device="cuda")
+    want = np.ascontiguousarray(wref[:, ks].T)
+    for odt in (torch.float32, tdt):
+        y = hk.gemm_w4a16_ws(x, torch.from_numpy(nib).cuda(), torch.from_numpy(sc).cuda(), n, k, ws,
+                             None if a is None else torch.from_numpy(a).cuda(), out_dtype=odt)
+        torch.cuda.synchronize()
+        assert np.array_equal(y.float().cpu().numpy(), want)
+
+
 def test_gemm_w4a16_ws_falls_back(orc, torch_dev, hk):
     """Up to M = 512 (no AWQ factors), or without a workspace, nve_hip_gemm_w4a16_ws is the fused kernel
     (compared at fp16 output: with a workspace an fp32 product at small M splits K, whose
