@@ -40,7 +40,7 @@ constexpr int kGemmBlasMinMAwq = 385;
 
 // Whether the tile kernel serves a product that dequant + GEMM could: its planned time against
 // 11.6 us + 0.635 us per 10^6 weights (the dequant and reading its output) + 0.573 us per GFLOP + 1.5 us
-// per 1000 of K, fitted to 364 timed products (12 layer shapes, N 512-14336, K 2048-14336, M =
+// per 1000 of K, fitted to 308 timed products (11 layer shapes, N 1024-14336, K 2048-14336, M =
 // 400-2048, with and without AWQ, fp16 and bf16; rms error 6%), with 8% for the estimates' error.
 // us, dequant + GEMM / tile kernel, fp16: 8B down M = 520 / 1024 112.8 / 91.6 and 148.1 / 122.7 (M = 1280
 // 163.1 / 182.6, stays), q 640 / 1024 40.5 / 32.8 and 47.1 / 39.8, 2048 x 2048 M = 1024 23.8 / 16.5; AWQ, M = 512,
